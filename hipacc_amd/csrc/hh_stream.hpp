@@ -28,7 +28,39 @@
 
 namespace hh {
 
-enum StreamKind { kStream2D = 0, kStreamSep = 1, kStreamBox = 2 };
+// kStreamMin / kStreamMax: the smallest / largest pixel of the window, row
+// extremes first, then the extreme of the KY rows (comparisons, so the row
+// and column passes may be split for any mask).
+enum StreamKind { kStream2D = 0, kStreamSep = 1, kStreamBox = 2, kStreamMin = 3, kStreamMax = 4 };
+constexpr bool stream_is_minmax(int kind) { return kind == kStreamMin || kind == kStreamMax; }
+
+// The running MIN / MAX keeps its value unless the tap is strictly smaller /
+// larger (reduce_combine): a equal to b keeps a, and a NaN tap never replaces.
+template <int KIND, typename ACC> __device__ __forceinline__ ACC stream_pick(ACC a, ACC b) {
+  if constexpr (KIND == kStreamMin) return b < a ? b : a;
+  else return b > a ? b : a;
+}
+
+// h[e] = extreme of v[e .. e + K - 1], by doubling (spans 1, 2, 4, ..., then
+// two overlapping spans): ceil(log2 K) picks per pixel instead of K - 1.  The
+// left span comes first, so ties keep the first pixel in row order.
+template <int KIND, int K, int V, int N, typename ACC>
+__device__ __forceinline__ void stream_row_extreme(const ACC (&v)[N], ACC (&h)[V]) {
+  ACC t[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) t[i] = v[i];
+  int span = 1;
+#pragma unroll
+  for (int lvl = 0; lvl < 4; ++lvl) {
+    if (2 * span > K) break;
+#pragma unroll
+    for (int i = 0; i + 2 * span <= N; ++i) t[i] = stream_pick<KIND>(t[i], t[i + span]);
+    span *= 2;
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e)
+    h[e] = span == K ? t[e] : stream_pick<KIND>(t[e], t[e + K - span]);
+}
 
 struct StreamGeom {
   int strips, segs, seg_rows;  // tiling of one image
@@ -196,6 +228,32 @@ __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw
         }
       }
     }
+  } else if constexpr (stream_is_minmax(KIND)) {
+    // Float taps that are NaN never replace the running value, whatever it
+    // is: they take part as the identity, except the window's first tap,
+    // which seeds the sequence and, when NaN, stays to the end.
+    ACC v[NWIN], h[V];
+#pragma unroll
+    for (int wi = 0; wi < NWIN; ++wi) {
+      if constexpr (IS_F) {
+        const ACC id = KIND == kStreamMin ? __builtin_huge_valf() : -__builtin_huge_valf();
+        v[wi] = win[wi] == win[wi] ? win[wi] : id;
+      } else {
+        v[wi] = win[wi];
+      }
+    }
+    stream_row_extreme<KIND, KX, V, NWIN, ACC>(v, h);
+#pragma unroll
+    for (int dyi = 0; dyi < KY; ++dyi) {
+      if (dyi > maxdy) break;
+      if (dyi < mindy) continue;
+      const int s = (slot0 - dyi + KY) % KY;
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if (dyi == 0) acc[s][e] = IS_F && !(win[e] == win[e]) ? win[e] : h[e];
+        else acc[s][e] = stream_pick<KIND>(acc[s][e], h[e]);
+      }
+    }
   } else {
     ACC h[V];
     if constexpr (KIND == kStreamBox) {
@@ -279,7 +337,8 @@ __device__ __forceinline__ void stream_block(const ArgsT& a, const StreamCtx<TI,
                                              TI (&ring)[PF][V], ACC (&acc)[KY][V], const TI* base,
                                              TO* orow, bool full, bool any, float rnd, int jb) {
   const Geom& g = a.g;
-  const bool cmode_sep = KIND != kStream2D && !FAST && g.boundary == HIPACC_BOUNDARY_CONSTANT;
+  const bool cmode_sep = (KIND == kStreamSep || KIND == kStreamBox) && !FAST &&
+                         g.boundary == HIPACC_BOUNDARY_CONSTANT;
   // every refill of this block is in range (always for the non-tail blocks)
   const bool full_blk = !TAIL || jb + 2 * PF <= c.nj;
 #pragma unroll

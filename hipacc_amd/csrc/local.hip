@@ -136,7 +136,11 @@ int launch_local(const LocalArgs& a, int acc_is_float, hipStream_t s, int varian
     if (!a.use_weights) fast = false;
   }
   if (variant == kVarGeneric) return launch_generic(a, acc_is_float, s);
-  if (!fast) return variant == kVarAuto ? launch_generic(a, acc_is_float, s) : HIPACC_ERR_UNSUPPORTED;
+  if (!fast) {
+    if (variant != kVarAuto) return HIPACC_ERR_UNSUPPORTED;
+    const int st = dispatch_stream_minmax(a, acc_is_float, 0, s);
+    return st == HIPACC_ERR_UNSUPPORTED ? launch_generic(a, acc_is_float, s) : st;
+  }
   LocalArgs f = a;
   const int n = a.mask_w * a.mask_h;
   for (int t = 0; t < n; ++t) {
