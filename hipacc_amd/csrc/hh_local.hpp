@@ -106,6 +106,7 @@ int launch_separable(const SepArgs& a, int acc_is_float, int fp_contract,
                      hipStream_t stream, int variant, int param);
 int dispatch_stream_local(const LocalArgs& a, int acc_is_float, int seg, int wide, hipStream_t s);
 int dispatch_stream_minmax(const LocalArgs& a, int acc_is_float, int seg, hipStream_t s);
+int dispatch_stream_vec4(const LocalArgs& a, int acc_is_float, hipStream_t s);
 int dispatch_ring_local(const LocalArgs& a, int seg_rows, hipStream_t s);
 int dispatch_ring8_local(const LocalArgs& a, int acc_is_float, int seg_rows, hipStream_t s);
 bool ring8_pays(const LocalArgs& a);

@@ -41,10 +41,10 @@ template <int KIND, typename ACC> __device__ __forceinline__ ACC stream_pick(ACC
   else return b > a ? b : a;
 }
 
-// h[e] = extreme of v[e .. e + K - 1], by doubling (spans 1, 2, 4, ..., then
+// h[e] = extreme of v[e], v[e + CH], ..., v[e + (K - 1) CH], by doubling (spans 1, 2, 4, ..., then
 // two overlapping spans): ceil(log2 K) picks per pixel instead of K - 1.  The
 // left span comes first, so ties keep the first pixel in row order.
-template <int KIND, int K, int V, int N, typename ACC>
+template <int KIND, int K, int V, int N, int CH, typename ACC>
 __device__ __forceinline__ void stream_row_extreme(const ACC (&v)[N], ACC (&h)[V]) {
   ACC t[N];
 #pragma unroll
@@ -54,12 +54,13 @@ __device__ __forceinline__ void stream_row_extreme(const ACC (&v)[N], ACC (&h)[V
   for (int lvl = 0; lvl < 4; ++lvl) {
     if (2 * span > K) break;
 #pragma unroll
-    for (int i = 0; i + 2 * span <= N; ++i) t[i] = stream_pick<KIND>(t[i], t[i + span]);
+    for (int i = 0; i + (2 * span - 1) * CH < N; ++i)
+      t[i] = stream_pick<KIND>(t[i], t[i + span * CH]);
     span *= 2;
   }
 #pragma unroll
   for (int e = 0; e < V; ++e)
-    h[e] = span == K ? t[e] : stream_pick<KIND>(t[e], t[e + K - span]);
+    h[e] = span == K ? t[e] : stream_pick<KIND>(t[e], t[e + (K - span) * CH]);
 }
 
 struct StreamGeom {
@@ -98,7 +99,9 @@ template <int V> struct LaneCols {
   bool cst[V];
 };
 
-template <int V> __device__ __forceinline__ LaneCols<V> lane_cols(const Geom& g, int ix) {
+// CH = 4: columns are the interleaved channels of 4-wide pixels; the map
+// applies to the pixel and keeps the channel.
+template <int V, int CH = 1> __device__ __forceinline__ LaneCols<V> lane_cols(const Geom& g, int ix) {
   LaneCols<V> c;
   const bool cmode = g.boundary == HIPACC_BOUNDARY_CONSTANT;
 #pragma unroll
@@ -109,7 +112,12 @@ template <int V> __device__ __forceinline__ LaneCols<V> lane_cols(const Geom& g,
       c.x[e] = c.cst[e] ? g.lo_x : x;
     } else {
       c.cst[e] = false;
-      c.x[e] = bh_map(g.boundary, x, g.lo_x, g.hi_x, g.in_imgw);
+      if constexpr (CH == 1) {
+        c.x[e] = bh_map(g.boundary, x, g.lo_x, g.hi_x, g.in_imgw);
+      } else {
+        static_assert(CH == 4, "channels");
+        c.x[e] = bh_map(g.boundary, x >> 2, g.lo_x >> 2, g.hi_x >> 2, g.in_imgw >> 2) * 4 + (x & 3);
+      }
     }
   }
   return c;
@@ -192,12 +200,14 @@ __device__ __forceinline__ void edge_row_load(TI (&v)[V], const Geom& g, const T
 // with mindy <= dyi <= maxdy exist: maxdy < KY-1 in the first rows of a
 // segment (a constant after unrolling, so the skipped taps cost nothing),
 // mindy > 0 in its last rows, past the segment's last output.
-template <typename TI, typename ACC, int V, int KX, int KY, bool FMA, int KIND, bool WDEV,
+// CH: distance of horizontally adjacent taps in row elements (4: the channels
+// of 4-wide pixels, each summed by itself).
+template <typename TI, typename ACC, int V, int KX, int KY, bool FMA, int KIND, bool WDEV, int CH,
           typename ArgsT>
 __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw)[V],
                                                   ACC (&acc)[KY][V], int slot0, bool cst_row,
                                                   int maxdy, int mindy) {
-  constexpr int RX = KX / 2;
+  constexpr int RX = KX / 2 * CH;
   constexpr int NWIN = V + 2 * RX;
   constexpr bool IS_F = std::is_same<ACC, float>::value;
   ACC cur[V];
@@ -224,7 +234,7 @@ __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw
         for (int e = 0; e < V; ++e) {
           // the first tap of an output starts its sum: round(w*x) == fma(w, x, 0)
           if (dyi == 0 && dx == 0) acc[s][e] = mul_first(w, win[e]);
-          else acc[s][e] = madd<FMA>(w, win[e + dx], acc[s][e]);
+          else acc[s][e] = madd<FMA>(w, win[e + dx * CH], acc[s][e]);
         }
       }
     }
@@ -242,7 +252,7 @@ __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw
         v[wi] = win[wi];
       }
     }
-    stream_row_extreme<KIND, KX, V, NWIN, ACC>(v, h);
+    stream_row_extreme<KIND, KX, V, NWIN, CH, ACC>(v, h);
 #pragma unroll
     for (int dyi = 0; dyi < KY; ++dyi) {
       if (dyi > maxdy) break;
@@ -304,7 +314,8 @@ __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw
 // streaming variants are only chosen without post_div and, for float
 // outputs, without rounding, so the conversion needs no division; full
 // vectors are written with nontemporal stores (the output is not re-read).
-template <typename TO, typename ACC, int V>
+// CH = 4 also takes post_div (the RGBA box blur).
+template <typename TO, typename ACC, int V, int CH>
 __device__ __forceinline__ void stream_store(TO* __restrict__ orow, const Geom& g, bool full,
                                              bool any, int xl, float rnd, const ACC (&acc)[V]) {
   if (!any) return;
@@ -317,6 +328,17 @@ __device__ __forceinline__ void stream_store(TO* __restrict__ orow, const Geom& 
       vals[e] = cvt_out<TO>::from_f((float)acc[e] + rnd);
     else
       vals[e] = cvt_out<TO>::from_i((int32_t)acc[e]);
+  }
+  if constexpr (CH == 4) {
+    if (g.post_div != 0.0f) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if constexpr (std::is_same<ACC, float>::value)
+          vals[e] = convert_f<TO>((float)acc[e], g.cvt, g.post_div);
+        else
+          vals[e] = convert_i<TO>((int32_t)acc[e], g.cvt, g.post_div);
+      }
+    }
   }
   TO* dst = orow + xl;
   if (full) {
@@ -332,7 +354,7 @@ __device__ __forceinline__ void stream_store(TO* __restrict__ orow, const Geom& 
 // accumulator slot are compile-time constants inside a block).  WARM: the
 // first block of the segment, whose row u only reaches outputs 0..u.
 template <typename TI, typename TO, typename ACC, int V, int KX, int KY, int PF, bool FMA,
-          int KIND, bool WDEV, bool FAST, bool WARM, bool TAIL, typename ArgsT>
+          int KIND, bool WDEV, int CH, bool FAST, bool WARM, bool TAIL, typename ArgsT>
 __device__ __forceinline__ void stream_block(const ArgsT& a, const StreamCtx<TI, TO, V>& c,
                                              TI (&ring)[PF][V], ACC (&acc)[KY][V], const TI* base,
                                              TO* orow, bool full, bool any, float rnd, int jb) {
@@ -362,11 +384,11 @@ __device__ __forceinline__ void stream_block(const ArgsT& a, const StreamCtx<TI,
     // where they are a fifth of the work or more; for small masks the extra
     // branches cost more than they save.
     constexpr bool SKIP_TAIL = TAIL && KY >= 7;
-    stream_accumulate<TI, ACC, V, KX, KY, FMA, KIND, WDEV>(a, raw, acc, u % KY, cst_row,
+    stream_accumulate<TI, ACC, V, KX, KY, FMA, KIND, WDEV, CH>(a, raw, acc, u % KY, cst_row,
                                                            WARM ? u : KY - 1,
                                                            SKIP_TAIL ? j - c.nj + KY : 0);
     if (!WARM || u >= KY - 1)
-      stream_store<TO, ACC, V>(orow + (long long)j * g.out_stride, g, full, any, c.xl, rnd,
+      stream_store<TO, ACC, V, CH>(orow + (long long)j * g.out_stride, g, full, any, c.xl, rnd,
                                acc[(u % KY + 1) % KY]);
   }
 }
@@ -376,7 +398,7 @@ __device__ __forceinline__ void stream_block(const ArgsT& a, const StreamCtx<TI,
 // the segment load unconditionally; the last blocks skip the refills past the
 // segment's last row (a wave-uniform branch).
 template <typename TI, typename TO, typename ACC, int V, int KX, int KY, int PF, bool FMA,
-          int KIND, bool WDEV, bool FAST, typename ArgsT>
+          int KIND, bool WDEV, int CH, bool FAST, typename ArgsT>
 __device__ __forceinline__ void stream_rows(const ArgsT& a, const StreamCtx<TI, TO, V>& c) {
   const Geom& g = a.g;
   const bool full = c.store_lane && a.out_vec_ok && c.xl + V <= g.is_w;
@@ -393,28 +415,28 @@ __device__ __forceinline__ void stream_rows(const ArgsT& a, const StreamCtx<TI, 
     if constexpr (FAST) load_px<TI, V>(ring[p], base + (long long)r * g.in_stride);
     else edge_row_load<TI, V>(ring[p], g, c.in, c.cols, c.iy0 + r);
   }
-  stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, FAST, true, true>(
+  stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, FAST, true, true>(
       a, c, ring, acc, base, orow, full, any, rnd, 0);
   if constexpr (KY >= 7) {
     // full blocks, then the tail blocks that skip the taps past the segment
     int jb = PF;
     for (; jb + 2 * PF <= c.nj; jb += PF)
-      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, FAST, false, false>(
+      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, FAST, false, false>(
           a, c, ring, acc, base, orow, full, any, rnd, jb);
     for (; jb < c.nj; jb += PF)
-      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, FAST, false, true>(
+      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, FAST, false, true>(
           a, c, ring, acc, base, orow, full, any, rnd, jb);
   } else {
     for (int jb = PF; jb < c.nj; jb += PF)
-      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, FAST, false, true>(
+      stream_block<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, FAST, false, true>(
           a, c, ring, acc, base, orow, full, any, rnd, jb);
   }
 }
 
 template <typename TI, typename TO, typename ACC, int V, int KX, int KY, int PF, bool FMA,
-          int KIND, bool WDEV, typename ArgsT>
+          int KIND, bool WDEV, int CH, typename ArgsT>
 __global__ __launch_bounds__(256) void stream_kernel(const ArgsT a, const StreamGeom sg) {
-  constexpr int RX = KX / 2, RY = KY / 2;
+  constexpr int RX = KX / 2 * CH, RY = KY / 2;
   constexpr int HL = (RX + V - 1) / V;          // halo lanes on each side
   static_assert(PF % KY == 0 && PF >= KY, "prefetch ring must be a multiple of KY");
 
@@ -450,10 +472,10 @@ __global__ __launch_bounds__(256) void stream_kernel(const ArgsT a, const Stream
   const bool fast = a.in_vec_ok && wx0 >= lx && wx0 + 64 * V <= hx && c.iy0 >= ly &&
                     c.iy0 + c.nj <= hy;
   if (fast) {
-    stream_rows<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, true>(a, c);
+    stream_rows<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, true>(a, c);
   } else {
-    c.cols = lane_cols<V>(g, c.ix);
-    stream_rows<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, false>(a, c);
+    c.cols = lane_cols<V, CH>(g, c.ix);
+    stream_rows<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, false>(a, c);
   }
 }
 
@@ -499,17 +521,18 @@ static inline dim3 stream_grid(StreamGeom& sg) {
   return dim3(blocks);
 }
 
+// CH = 4: the channel view of 4-wide pixels (columns and strides x 4).
 template <typename TI, typename TO, typename ACC, int V, int KX, int KY, int PF, bool FMA,
-          int KIND, bool WDEV, typename ArgsT>
+          int KIND, bool WDEV, int CH = 1, typename ArgsT>
 static int launch_stream(const ArgsT& a0, int seg_rows, hipStream_t s) {
-  if (a0.g.post_div != 0.0f ||
+  if ((CH == 1 && a0.g.post_div != 0.0f) ||
       (std::is_same<TO, float>::value && a0.g.cvt == HIPACC_CVT_ROUND))
     return HIPACC_ERR_UNSUPPORTED;
   ArgsT a = a0;
   stream_align(a.g, V, a.in_vec_ok, a.out_vec_ok);
-  StreamGeom sg = stream_geom(a.g, KX / 2, V, seg_rows);
+  StreamGeom sg = stream_geom(a.g, KX / 2 * CH, V, seg_rows);
   const dim3 grid = stream_grid(sg);
-  hipLaunchKernelGGL((stream_kernel<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, ArgsT>), grid,
+  hipLaunchKernelGGL((stream_kernel<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, ArgsT>), grid,
                      dim3(256), 0, s, a, sg);
   return hip_status(hipGetLastError(), "stream_kernel launch");
 }

@@ -124,9 +124,12 @@ static int launch_local_variant(const LocalArgs& f, int acc_is_float, hipStream_
 // A forced variant returns HIPACC_ERR_UNSUPPORTED when it has no kernel for
 // the operator's shape.
 int launch_local(const LocalArgs& a, int acc_is_float, hipStream_t s, int variant, int param) {
-  if (dtype_is_vec(a.g.in_dtype))
-    return variant == kVarAuto || variant == kVarGeneric ? launch_local_vec4(a, acc_is_float, s)
-                                                         : HIPACC_ERR_UNSUPPORTED;
+  if (dtype_is_vec(a.g.in_dtype)) {
+    if (variant != kVarAuto && variant != kVarGeneric) return HIPACC_ERR_UNSUPPORTED;
+    const int st =
+        variant == kVarAuto ? dispatch_stream_vec4(a, acc_is_float, s) : HIPACC_ERR_UNSUPPORTED;
+    return st == HIPACC_ERR_UNSUPPORTED ? launch_local_vec4(a, acc_is_float, s) : st;
+  }
   // The tile and stream kernels implement SUM with weights (or a full domain);
   // domain holes become zero weights, which leaves every finite sum unchanged.
   bool fast = a.reduce == HIPACC_REDUCE_SUM && a.mask_w == a.mask_h;
