@@ -1,0 +1,258 @@
+// bilat_pair.hip -- bilateral filter on float images, each pixel pair's
+// weight evaluated once (hh_bilat_pair.hpp).
+//
+// Per pair of pixels: difference, exponent (one FMA on pixels scaled by
+// sqrt(c log2 e)), exponential (two issue slots) and the four sums of the
+// pair, 8 slots; the tile kernel (bilateral.hip) spends 7 on each of the
+// pair's two taps.  The sums are of d = X(q) - X(p), so that
+// Y(p) = X(p) + SUM s d / SUM s: the rounding of the sums scales with the
+// local contrast instead of the pixel's value (13x13 over 4096^2 pixels in
+// [0, 1]: 3.5e-8 off the 64-bit result in the 2-norm, the tile kernel 2.8e-7).
+//
+// 4096^2: 13x13 527 -> 405 us, 7x7 175 -> 120 us; 16 x 1024^2 7x7 173 -> 126
+// us (tile kernel -> here); VALU issue bound, 2970 of 3120 slots of a 13x13
+// row in the pairs.
+#include <cmath>
+
+#include "hh_bilat_pair.hpp"
+
+namespace hh {
+
+typedef float pair_f4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int R>
+__global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const BilatArgs a, const PairGeom pg) {
+  constexpr int V = 4, K = 2 * R + 1, HL = (R + V - 1) / V, NW = V + 2 * R;
+  __shared__ __align__(16) float4 part[3][R][2][64];   // first R rows of waves 1..3: den, num
+  const Geom& g = a.g;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const PairLane pl = pair_lane<HL>(pg, lane, 3 * pg.n + pg.n0);
+  const float* in = static_cast<const float*>(g.in) + (long long)pl.b * g.in_plane;
+  const int yw = pl.y0 + (wave == 0 ? 0 : pg.n0 + (wave - 1) * pg.n);   // first row of the segment
+  const int nrow = wave == 0 ? pg.n0 : pg.n;
+  const bool cmode = g.boundary == HIPACC_BOUNDARY_CONSTANT;
+  const LaneCols<V> cols = lane_cols<V>(g, g.in_ox + pl.x);
+  bool raw = true;   // the lane's 4 pixels are adjacent in memory
+#pragma unroll
+  for (int e = 0; e < V; ++e) raw = raw && !cols.cst[e] && cols.x[e] == cols.x[0] + e;
+
+  const int lead = wave == 0 ? R : 0;      // rows walked above the segment
+  const int ys = yw - lead;                // first row walked
+  const int steps = nrow + lead;
+  // rows ys .. ys + steps + R + 1 are loaded
+  int lx, hx, ly, hy;
+  raw_region(g, lx, hx, ly, hy);
+  const bool walk = __all(raw && g.in_oy + ys >= ly && g.in_oy + ys + steps + R + 2 <= hy);
+  const float* next = in + (long long)(g.in_oy + ys) * g.in_stride + cols.x[0];
+
+  // Pixels of row y (iteration space), boundary handling applied; called for
+  // consecutive rows from ys on.
+  auto load_row = [&](int y, float (&v)[V]) {
+    if (walk) {
+      const pair_f4 q = *reinterpret_cast<const pair_f4*>(next);
+      next += g.in_stride;
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = q[e];
+      return;
+    }
+    bool rc;
+    const int yy = row_src(g, g.in_oy + y, rc);
+    const float* row = in + (long long)yy * g.in_stride;
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = row[cols.x[e]];
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = rc || cols.cst[e] ? g.const_f : v[e];
+  };
+
+  float ref = 0.0f;                        // pixels are scaled about this value
+  const float sc = __builtin_sqrtf(-a.k2), isc = 1.0f / sc;
+  const float s0 = __builtin_amdgcn_exp2f(a.lsp[R * K + R]);
+  // x, den, num: scaled pixels of row y and their sums (without the centre tap)
+  auto finish = [&](int y, const float (&x)[V], const float (&den)[V], const float (&num)[V]) {
+    if (!pl.store || y >= g.is_h) return;
+    float r[V], n[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      n[e] = den[e] + s0;
+      // with a centre weight the sum is no denormal and the reciprocal's last
+      // bit only scales the correction SUM s d / SUM s
+      const float q = s0 > 1e-30f ? num[e] * __builtin_amdgcn_rcpf(n[e]) : num[e] / n[e];
+      r[e] = __builtin_fmaf(x[e] + q, isc, ref);
+    }
+    float* dst = static_cast<float*>(g.out) + (long long)pl.b * g.out_plane +
+                 (long long)(g.out_oy + y) * g.out_stride + g.out_ox + pl.x;
+    float* nrm = a.norm ? a.norm + (long long)pl.b * a.norm_plane +
+                              (long long)y * a.norm_stride + pl.x
+                        : nullptr;
+    if (pl.x + V <= g.is_w) {
+      pair_f4 q = {r[0], r[1], r[2], r[3]};
+      __builtin_nontemporal_store(q, reinterpret_cast<pair_f4*>(dst));
+      if (nrm) {
+        pair_f4 m = {n[0], n[1], n[2], n[3]};
+        __builtin_nontemporal_store(m, reinterpret_cast<pair_f4*>(nrm));
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        if (pl.x + e < g.is_w) {
+          dst[e] = r[e];
+          if (nrm) nrm[e] = n[e];
+        }
+    }
+  };
+
+  float xr[R + 1][V], nx[V];               // rows y .. y + R, scaled; row y + R + 1 as loaded
+  float den[R + 1][V], num[R + 1][V];      // sums of rows y .. y + R
+  auto scaled = [&](const float (&v)[V], float (&x)[V]) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e] = (v[e] - ref) * sc;
+  };
+  {
+    float v[R + 1][V];
+#pragma unroll
+    for (int k = 0; k <= R; ++k) load_row(ys + k, v[k]);
+    load_row(ys + R + 1, nx);
+    const float f = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v[0][0])));
+    ref = __builtin_fabsf(f) < 1e30f ? f : 0.0f;
+#pragma unroll
+    for (int k = 0; k <= R; ++k) {
+      scaled(v[k], xr[k]);
+#pragma unroll
+      for (int e = 0; e < V; ++e) den[k][e] = num[k][e] = 0.0f;
+    }
+  }
+#pragma unroll 1
+  for (int r = 0; r < steps; ++r) {
+    const int y = ys + r;
+    if (!__any(y < g.is_h)) break;         // the rest of the band is below the image
+    float nn[V];
+    load_row(y + R + 2, nn);
+#pragma unroll
+    for (int dy = 0; dy <= R; ++dy) {
+      if (r + dy < lead) continue;         // pairs of rows above the segment
+      // The window of row y + dy slides over the offsets: its element m is
+      // first used at dx = m - R - 3 and its sums are complete after
+      // dx = m - R, when they go to the lane that owns the column.
+      float win[NW], wd[NW], wn[NW];
+      auto column = [](int m, int& d, int& e) {
+        const int rel = m - R;
+        d = rel >= 0 ? rel / V : -((-rel + V - 1) / V);
+        e = rel - d * V;
+      };
+      const int first = dy == 0 ? 1 : -R;
+#pragma unroll
+      for (int dx = first; dx <= R; ++dx) {
+        const float l = a.lsp[(R + dy) * K + R + dx];
+#pragma unroll
+        for (int m = dx == first ? dx + R : dx + R + V - 1; m < dx + R + V; ++m) {
+          int d, e;
+          column(m, d, e);
+          win[m] = lane_shift(xr[dy][e], d);
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          const int m = e + dx + R;
+          const float d = win[m] - xr[0][e];
+          const float s = __builtin_amdgcn_exp2f(__builtin_fmaf(-d, d, l));
+          den[0][e] += s;
+          num[0][e] = __builtin_fmaf(s, d, num[0][e]);
+          if (dx == first || e == V - 1) {
+            wd[m] = s;
+            wn[m] = -s * d;
+          } else {
+            wd[m] += s;
+            wn[m] = __builtin_fmaf(-s, d, wn[m]);
+          }
+        }
+        // (one offset later: a DPP read right after the write would wait)
+#pragma unroll
+        for (int m = dx == first ? NW : dx + R - 1; m < (dx == R ? NW : dx + R); ++m) {
+          int d, e;
+          column(m, d, e);
+          den[dy][e] += lane_shift(wd[m], -d);
+          num[dy][e] += lane_shift(wn[m], -d);
+          asm volatile("" : "+v"(den[dy][e]), "+v"(num[dy][e]));
+        }
+        // the sums are pinned per offset: left alone, the compiler sinks
+        // their additions past the row and keeps hundreds of weights live
+        // (9x9: 119 registers against more than 256)
+#pragma unroll
+        for (int e = 0; e < V; ++e) asm volatile("" : "+v"(den[0][e]), "+v"(num[0][e]));
+      }
+    }
+    const int rs = r - lead;               // row of the segment
+    if (rs >= 0) {
+      if (wave > 0 && rs < R) {
+        part[wave - 1][rs][0][lane] = make_float4(den[0][0], den[0][1], den[0][2], den[0][3]);
+        part[wave - 1][rs][1][lane] = make_float4(num[0][0], num[0][1], num[0][2], num[0][3]);
+      } else {
+        finish(y, xr[0], den[0], num[0]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        xr[k][e] = xr[k + 1][e];
+        den[k][e] = den[k + 1][e];
+        num[k][e] = num[k + 1][e];
+      }
+    scaled(nx, xr[R]);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      nx[e] = nn[e];
+      den[R][e] = num[R][e] = 0.0f;
+    }
+  }
+  __syncthreads();
+  if (wave < 3) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const float4 pd = part[wave][k][0][lane], pn = part[wave][k][1][lane];
+      const float d[V] = {den[k][0] + pd.x, den[k][1] + pd.y, den[k][2] + pd.z, den[k][3] + pd.w};
+      const float m[V] = {num[k][0] + pn.x, num[k][1] + pn.y, num[k][2] + pn.z, num[k][3] + pn.w};
+      finish(yw + nrow + k, xr[k], d, m);
+    }
+  }
+}
+
+int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 256;
+    return n;
+  }();
+  const Geom& g = a.g;
+  if (g.in_dtype != HIPACC_F32 || g.out_dtype != HIPACC_F32 || g.cvt == HIPACC_CVT_ROUND)
+    return HIPACC_ERR_UNSUPPORTED;
+  const int kk = a.ksize * a.ksize, r = a.ksize / 2;
+  for (int t = 0; t < kk; ++t)
+    if (!(a.lsp[t] == a.lsp[kk - 1 - t])) return HIPACC_ERR_UNSUPPORTED;
+  const PairGeom pg = pair_geom(g.is_w, g.is_h, g.batch, r, cus);
+  if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
+  // Issue slots of a SIMD, both ways: a tile block is one wave per SIMD of 4
+  // pixels x 7 slots a tap, a row of this kernel 4 pixels x 8.9 slots a pair
+  // (both plus staging).  The long segments of this kernel lose where the
+  // image does not fill the device a few times over: 7x7 at 1001x751 13.2
+  // (tile) and 15.7 us, at 1920x1080 36 and 27 us; 13x13 at 1024^2 39 and 43
+  // us, at 1920x1080 72 and 68 us.
+  const double tile = (double)ceil_div(ceil_div(g.is_w, 64) * ceil_div(g.is_h, 16) * g.batch, cus) *
+                      (28.0 * kk + 300.0);
+  const double pair = (double)ceil_div(pg.blocks, cus) * (pg.n + 1.5) * (17.8 * kk + 180.0);
+  if (tile < pair) return HIPACC_ERR_UNSUPPORTED;
+#define HH_BP(R)                                                                             \
+  case R:                                                                                    \
+    hipLaunchKernelGGL((bilat_pair_kernel<R>), dim3(pg.blocks), dim3(256), 0, s, a, pg);     \
+    break;
+  switch (r) {
+    HH_BP(2) HH_BP(3) HH_BP(4) HH_BP(5) HH_BP(6) HH_BP(7)
+    default: return HIPACC_ERR_UNSUPPORTED;
+  }
+#undef HH_BP
+  return hip_status(hipGetLastError(), "bilat_pair_kernel launch");
+}
+
+}  // namespace hh

@@ -122,6 +122,8 @@ static int launch_bilat_t(const BilatArgs& a, hipStream_t s) {
 }
 
 int launch_bilateral(const BilatArgs& a, hipStream_t s) {
+  const int st = dispatch_bilat_pair(a, s);
+  if (st != HIPACC_ERR_UNSUPPORTED) return st;
   const bool f = a.g.in_dtype == HIPACC_F32;
 #define HH_BIL(K)                                                              \
   case K:                                                                      \

@@ -172,6 +172,8 @@ struct BilatArgs {
   int norm_stride;
 };
 int launch_bilateral(const BilatArgs& a, hipStream_t s);
+// Float images through the pixel-pair kernel (bilat_pair.hip).
+int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s);
 
 // Records the detailed message of the calling thread's last failure.
 int set_error(int status, const char* fmt, ...);
