@@ -235,13 +235,15 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   // Issue slots of a SIMD, both ways: a tile block is one wave per SIMD of 4
   // pixels x 7 slots a tap, a row of this kernel 4 pixels x 8.9 slots a pair
-  // (both plus staging).  The long segments of this kernel lose where the
-  // image does not fill the device a few times over: 7x7 at 1001x751 13.2
-  // (tile) and 15.7 us, at 1920x1080 36 and 27 us; 13x13 at 1024^2 39 and 43
-  // us, at 1920x1080 72 and 68 us.
+  // (both plus staging), and its first rows' loads are waited for.  The long
+  // segments lose where the image does not fill the device a few times over
+  // (us, tile and pair): 7x7 at 1001x751 13.1 and 14.2, at 1920x1080 24.0 and
+  // 24.4, at 2048^2 46 and 36.5; 13x13 at 1024^2 38 and 41, at 1920x1080 69
+  // and 64, at 2048^2 136 and 113.
   const double tile = (double)ceil_div(ceil_div(g.is_w, 64) * ceil_div(g.is_h, 16) * g.batch, cus) *
                       (28.0 * kk + 300.0);
-  const double pair = (double)ceil_div(pg.blocks, cus) * (pg.n + 1.5) * (17.8 * kk + 180.0);
+  const double pair =
+      (double)ceil_div(pg.blocks, cus) * (pg.n + 1.0) * (17.8 * kk + 180.0) + 2500.0;
   if (tile < pair) return HIPACC_ERR_UNSUPPORTED;
 #define HH_BP(R)                                                                             \
   case R:                                                                                    \

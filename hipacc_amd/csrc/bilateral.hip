@@ -33,21 +33,36 @@ __global__ __launch_bounds__(256) void bilateral_kernel(const BilatArgs a) {
   TO* out = static_cast<TO*>(g.out) + (long long)blockIdx.z * g.out_plane;
   const int ix0 = g.in_ox + tx0 - HV * VEC, iy0 = g.in_oy + ty0 - R;
   if constexpr (std::is_same<TI, float>::value) {
-    stage_tile<float, VEC, NV, LH>(tile, in, g, ix0, iy0, a.in_vec_ok);
+    stage_tile<float, VEC, NV, LH>(tile, in, g, ix0, iy0);
+  } else if (raw_tile(g, ix0, iy0, LW, LH)) {
+    // uchar images are widened to float while staging, 4 pixels a load
+    constexpr int N = LH * NV, NL = (N + 255) / 256;
+    const TI* src = in + (long long)iy0 * g.in_stride + ix0;
+    unsigned w[NL];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int i = min((int)threadIdx.x + k * 256, N - 1);
+      const int r = i / NV;
+      w[k] = *reinterpret_cast<const u32_any*>(src + (long long)r * g.in_stride + (i - r * NV) * VEC);
+    }
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int i = threadIdx.x + k * 256;
+      if (i < N)
+        reinterpret_cast<float4*>(tile)[i] =
+            make_float4((float)(w[k] & 0xffu), (float)((w[k] >> 8) & 0xffu),
+                        (float)((w[k] >> 16) & 0xffu), (float)(w[k] >> 24));
+    }
   } else {
-    // uchar images are widened to float while staging (per element).
     const bool cmode = g.boundary == HIPACC_BOUNDARY_CONSTANT;
-    int lx, hx, ly, hy;
-    raw_region(g, lx, hx, ly, hy);
-    const bool interior = ix0 >= lx && ix0 + LW <= hx && iy0 >= ly && iy0 + LH <= hy;
     for (int i = threadIdx.x; i < LH * LW; i += 256) {
       const int r = i / LW, c = i - r * LW;
       int x = ix0 + c, y = iy0 + r;
       float v;
-      if (!interior && cmode && (x < g.lo_x || x >= g.hi_x || y < g.lo_y || y >= g.hi_y)) {
+      if (cmode && (x < g.lo_x || x >= g.hi_x || y < g.lo_y || y >= g.hi_y)) {
         v = (float)(TI)g.const_i;
       } else {
-        if (!interior && !cmode) {
+        if (!cmode) {
           x = bh_map(g.boundary, x, g.lo_x, g.hi_x, g.in_imgw);
           y = bh_map(g.boundary, y, g.lo_y, g.hi_y, g.in_imgh);
         }

@@ -39,7 +39,7 @@ struct LocalArgs {
   int reduce;
   int use_weights;
   int fma;          // fp_contract
-  int in_vec_ok;    // input window admits aligned 16-byte row loads
+  int in_vec_ok;    // input window admits aligned 16-byte row loads (direct loads to LDS)
   int out_vec_ok;   // output window admits aligned vector stores
   const float* wdev;
   uint8_t domain[kMaxTaps];
@@ -125,7 +125,7 @@ struct PointArgs {
   int w, h, batch;
   int op, cvt;
   float alpha, beta;
-  int vec_ok;
+  int vec_ok;   // output vectors are aligned (set at the launch)
 };
 int launch_point(const PointArgs& a, int dt0, int dt1, int dto, hipStream_t s);
 

@@ -99,9 +99,11 @@ __device__ __forceinline__ float4 ring_merge(const float4& a, const float4& b) {
 // The block computes output rows [y0, y0 + nout) of its strip; xl is the
 // iteration-space column of the lane's first pixel.  CH rows per LDS chunk.
 // Interior strips stage their rows with direct global->LDS loads, ND chunks
-// ahead, through a ring of ND+2 chunks; edge strips stage through NS
-// register sets and a ring of three chunks.
-template <int K, bool FMA, bool WDEV, int CH, int NS, int ND, bool EDGE>
+// ahead, through a ring of ND+2 chunks (DIRECT; 16-byte aligned rows, no row
+// outside a CONSTANT window); the others stage through NS register sets and
+// a ring of three chunks, interior strips with one 16-byte load per row at
+// whatever alignment the rows have.
+template <int K, bool FMA, bool WDEV, int CH, int NS, int ND, bool EDGE, bool DIRECT>
 __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict__ lds,
                                           const float* __restrict__ in, float* __restrict__ out,
                                           int xl, int y0, int nout) {
@@ -113,7 +115,8 @@ __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict
   // the larger masks, whose VALU work hides the per-pixel loads, keep the
   // registers and load every pixel of an edge strip separately.
   constexpr bool SPLIT = EDGE && K <= 5;
-  constexpr int NSLOT = EDGE ? 3 : ND + 2;   // chunks in the LDS ring
+  static_assert(!(EDGE && DIRECT), "edge strips have no direct loads");
+  constexpr int NSLOT = DIRECT ? ND + 2 : 3;   // chunks in the LDS ring
   const Geom& g = a.g;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
@@ -131,7 +134,7 @@ __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict
   if constexpr (EDGE) {
     int lx, hx, ly, hy;
     raw_region(g, lx, hx, ly, hy);
-    const bool lane_raw = SPLIT && a.in_vec_ok && ix >= lx && ix + V <= hx;
+    const bool lane_raw = SPLIT && ix >= lx && ix + V <= hx;
     // lanes farther than R columns from every stored column feed no output
     // (the iteration space ends inside the strip): they load nothing
     const int s0 = xl - lane * V + V, s1 = min(s0 + kRingStripW, g.is_w);
@@ -157,7 +160,7 @@ __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict
       st.rc |= rc ? 1 << i : 0;
       const float* row = in + (long long)y * g.in_stride;
       if constexpr (!EDGE) {
-        st.r[i] = *reinterpret_cast<const float4*>(row + ix);
+        st.r[i] = __builtin_bit_cast(float4, *reinterpret_cast<const u32x4_any*>(row + ix));
       } else {
         const __amdgpu_buffer_rsrc_t rs = ring_rsrc(row, in_row_bytes);
         float v[V];
@@ -201,7 +204,7 @@ __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict
   // iteration space (interior strips: every stored lane), else one 4-byte
   // store per pixel inside it
   const bool store_lane = lane >= 1 && lane < 63;
-  const bool full = store_lane && (!EDGE || (a.out_vec_ok && xl + V <= g.is_w));
+  const bool full = store_lane && (!EDGE || xl + V <= g.is_w);
   const int voff = full ? xl * 4 : kRingDrop;
   int soff[V];
   if constexpr (EDGE) {
@@ -286,7 +289,7 @@ __device__ __forceinline__ void ring_body(const LocalArgs& a, float4* __restrict
   };
 
   const int nos = (nout + CH - 1) / CH;
-  if constexpr (!EDGE) {
+  if constexpr (DIRECT) {
     // Direct loads: chunk c lands in slot c % NSLOT.  Step s waits for its
     // own loads of chunk s+1, meets the other waves at the barrier, issues
     // the loads of chunk s+ND+1 into the slot chunk s-1 held, and computes
@@ -400,19 +403,22 @@ __global__ __launch_bounds__(256) void ring_kernel(const LocalArgs a, const Ring
   int lx, hx, ly, hy;
   raw_region(g, lx, hx, ly, hy);
   const int ix0 = g.in_ox + xs;
-  // interior: raw columns, full vector stores, and (CONSTANT) no row outside
-  // the window -- the direct loads cannot substitute the constant
+  // interior: raw columns and full vector stores; the direct loads need
+  // aligned rows and cannot substitute the constant for a row outside the
+  // window
   const int iy0 = g.in_oy + it.y0 - K / 2;
-  const bool raw = a.in_vec_ok && a.out_vec_ok && ix0 >= lx && ix0 + 64 * kRingV <= hx &&
-                   xs + 63 * kRingV <= g.is_w &&
-                   (g.boundary != HIPACC_BOUNDARY_CONSTANT ||
-                    (iy0 >= g.lo_y && iy0 + it.nout + K - 1 <= g.hi_y));
-  if (raw)
-    ring_body<K, FMA, WDEV, CH, NS, ND, false>(a, lds, in, out, xs + lane * kRingV, it.y0,
-                                               it.nout);
+  const bool raw = ix0 >= lx && ix0 + 64 * kRingV <= hx && xs + 63 * kRingV <= g.is_w;
+  const bool direct = a.in_vec_ok && (g.boundary != HIPACC_BOUNDARY_CONSTANT ||
+                                      (iy0 >= g.lo_y && iy0 + it.nout + K - 1 <= g.hi_y));
+  if (raw && direct)
+    ring_body<K, FMA, WDEV, CH, NS, ND, false, true>(a, lds, in, out, xs + lane * kRingV, it.y0,
+                                                     it.nout);
+  else if (raw)
+    ring_body<K, FMA, WDEV, CH, NS, ND, false, false>(a, lds, in, out, xs + lane * kRingV, it.y0,
+                                                      it.nout);
   else
-    ring_body<K, FMA, WDEV, CH, NS, ND, true>(a, lds, in, out, xs + lane * kRingV, it.y0,
-                                              it.nout);
+    ring_body<K, FMA, WDEV, CH, NS, ND, true, false>(a, lds, in, out, xs + lane * kRingV, it.y0,
+                                                     it.nout);
 }
 
 // ---------------------------------------------------------------------------
@@ -490,8 +496,8 @@ __device__ __forceinline__ void ring_sep_body(const SepArgs& a, float4* __restri
       st.rc |= rc ? 1 << i : 0;
       const TI* row = in + (long long)y * g.in_stride;
       if constexpr (!EDGE) {
-        if constexpr (U8) st.r[i] = *reinterpret_cast<const unsigned*>(row + ix);
-        else st.r[i] = *reinterpret_cast<const float4*>(row + ix);
+        if constexpr (U8) st.r[i] = *reinterpret_cast<const u32_any*>(row + ix);
+        else st.r[i] = __builtin_bit_cast(float4, *reinterpret_cast<const u32x4_any*>(row + ix));
       } else {
         const __amdgpu_buffer_rsrc_t rs = ring_rsrc(row, in_row_bytes);
         if constexpr (U8) {
@@ -558,7 +564,11 @@ __device__ __forceinline__ void ring_sep_body(const SepArgs& a, float4* __restri
   };
 
   const bool store_lane = lane >= HL && lane < 64 - HL;
-  const bool full = store_lane && (!EDGE || (a.out_vec_ok && xl + V <= g.is_w));
+  // buffer stores need 4-byte alignment, which only 4-byte pixels always
+  // have: narrower pixels of unaligned rows take global stores (interior
+  // strips) or one store per pixel
+  const bool word_ok = BO == 4 || a.out_vec_ok;
+  const bool full = store_lane && (!EDGE || (word_ok && xl + V <= g.is_w));
   const int voff = full ? xl * BO : kRingDrop;
   int soff[V];
   if constexpr (EDGE) {
@@ -615,7 +625,8 @@ __device__ __forceinline__ void ring_sep_body(const SepArgs& a, float4* __restri
           unsigned w = 0;
 #pragma unroll
           for (int e = 0; e < V; ++e) w |= (unsigned)(uint8_t)px[e] << (8 * e);
-          __builtin_amdgcn_raw_buffer_store_b32(w, rs, voff, 0, 2);
+          if (EDGE || word_ok) __builtin_amdgcn_raw_buffer_store_b32(w, rs, voff, 0, 2);
+          else if (full && j < nout) store_vec<TO, V>(obase + (long long)j * g.out_stride + xl, px, false);
           if constexpr (EDGE) {
 #pragma unroll
             for (int e = 0; e < V; ++e)
@@ -625,7 +636,8 @@ __device__ __forceinline__ void ring_sep_body(const SepArgs& a, float4* __restri
           typedef unsigned int ring_u2 __attribute__((ext_vector_type(2)));
           const ring_u2 v = {(unsigned)(uint16_t)px[0] | (unsigned)(uint16_t)px[1] << 16,
                              (unsigned)(uint16_t)px[2] | (unsigned)(uint16_t)px[3] << 16};
-          __builtin_amdgcn_raw_buffer_store_b64(v, rs, voff, 0, 2);
+          if (EDGE || word_ok) __builtin_amdgcn_raw_buffer_store_b64(v, rs, voff, 0, 2);
+          else if (full && j < nout) store_vec<TO, V>(obase + (long long)j * g.out_stride + xl, px, false);
           if constexpr (EDGE) {
 #pragma unroll
             for (int e = 0; e < V; ++e)
@@ -692,8 +704,7 @@ __global__ __launch_bounds__(256) void ring_sep_kernel(const SepArgs a, const Ri
   int lx, hx, ly, hy;
   raw_region(g, lx, hx, ly, hy);
   const int ix0 = g.in_ox + xs;
-  const bool raw = a.in_vec_ok && a.out_vec_ok && ix0 >= lx && ix0 + 64 * kRingV <= hx &&
-                   xs + (64 - HL) * kRingV <= g.is_w;
+  const bool raw = ix0 >= lx && ix0 + 64 * kRingV <= hx && xs + (64 - HL) * kRingV <= g.is_w;
   if (raw)
     ring_sep_body<TI, TO, KX, KY, FMA, ISUM, false, CH, NS>(a, lds, in, out, xs + lane * kRingV,
                                                             it.y0, it.nout);

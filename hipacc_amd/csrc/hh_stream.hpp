@@ -147,20 +147,26 @@ template <> struct StreamTaps<LocalArgs> {
   }
 };
 
-// V pixels of T: loaded in 16-byte pieces (or one smaller word).
+// V pixels of T at any alignment: loaded in 16-byte pieces (or one smaller
+// word).
 template <typename T, int V>
 __device__ __forceinline__ void load_px(T (&v)[V], const T* p) {
   constexpr int B = V * (int)sizeof(T);
   if constexpr (B >= 16) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int k = 0; k < B / 16; ++k) {
-      const uint4 w = reinterpret_cast<const uint4*>(p)[k];
+      const u32x4 w = reinterpret_cast<const u32x4_any*>(p)[k];
       __builtin_memcpy(reinterpret_cast<char*>(v) + 16 * k, &w, 16);
     }
+  } else if constexpr (B == 8) {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 w = *reinterpret_cast<const u32x2_any*>(p);
+    __builtin_memcpy(v, &w, 8);
   } else {
-    using W = typename word_of<B>::type;
-    const W w = *reinterpret_cast<const W*>(p);
-    __builtin_memcpy(v, &w, B);
+    static_assert(B == 4, "pixel vector");
+    const unsigned int w = *reinterpret_cast<const u32_any*>(p);
+    __builtin_memcpy(v, &w, 4);
   }
 }
 
@@ -317,7 +323,8 @@ __device__ __forceinline__ void stream_accumulate(const ArgsT& a, const TI (&raw
 // CH = 4 also takes post_div (the RGBA box blur).
 template <typename TO, typename ACC, int V, int CH>
 __device__ __forceinline__ void stream_store(TO* __restrict__ orow, const Geom& g, bool full,
-                                             bool any, int xl, float rnd, const ACC (&acc)[V]) {
+                                             bool any, bool aligned, int xl, float rnd,
+                                             const ACC (&acc)[V]) {
   if (!any) return;
   TO vals[V];
 #pragma unroll
@@ -342,7 +349,7 @@ __device__ __forceinline__ void stream_store(TO* __restrict__ orow, const Geom& 
   }
   TO* dst = orow + xl;
   if (full) {
-    store_vec<TO, V>(dst, vals);
+    store_vec<TO, V>(dst, vals, aligned);
   } else {
 #pragma unroll
     for (int e = 0; e < V; ++e)
@@ -388,8 +395,8 @@ __device__ __forceinline__ void stream_block(const ArgsT& a, const StreamCtx<TI,
                                                            WARM ? u : KY - 1,
                                                            SKIP_TAIL ? j - c.nj + KY : 0);
     if (!WARM || u >= KY - 1)
-      stream_store<TO, ACC, V, CH>(orow + (long long)j * g.out_stride, g, full, any, c.xl, rnd,
-                               acc[(u % KY + 1) % KY]);
+      stream_store<TO, ACC, V, CH>(orow + (long long)j * g.out_stride, g, full, any,
+                                   a.out_vec_ok, c.xl, rnd, acc[(u % KY + 1) % KY]);
   }
 }
 
@@ -401,7 +408,7 @@ template <typename TI, typename TO, typename ACC, int V, int KX, int KY, int PF,
           int KIND, bool WDEV, int CH, bool FAST, typename ArgsT>
 __device__ __forceinline__ void stream_rows(const ArgsT& a, const StreamCtx<TI, TO, V>& c) {
   const Geom& g = a.g;
-  const bool full = c.store_lane && a.out_vec_ok && c.xl + V <= g.is_w;
+  const bool full = c.store_lane && c.xl + V <= g.is_w;
   const bool any = c.store_lane && c.xl < g.is_w;
   const float rnd = g.cvt == HIPACC_CVT_ROUND ? 0.5f : 0.0f;
   TO* orow = c.out + (long long)(g.out_oy + c.y0 - (KY - 1)) * g.out_stride + g.out_ox;
@@ -469,7 +476,7 @@ __global__ __launch_bounds__(256) void stream_kernel(const ArgsT a, const Stream
   raw_region(g, lx, hx, ly, hy);
   // The wave reads raw rows iy0 .. iy0+nj-1 and the columns of all 64 lanes.
   const int wx0 = g.in_ox + strip * sg.strip_w - HL * V;
-  const bool fast = a.in_vec_ok && wx0 >= lx && wx0 + 64 * V <= hx && c.iy0 >= ly &&
+  const bool fast = wx0 >= lx && wx0 + 64 * V <= hx && c.iy0 >= ly &&
                     c.iy0 + c.nj <= hy;
   if (fast) {
     stream_rows<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, true>(a, c);

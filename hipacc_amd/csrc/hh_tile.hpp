@@ -25,29 +25,45 @@ template <> struct word_of<4> { using type = uint32_t; };
 template <> struct word_of<8> { using type = uint2; };
 template <> struct word_of<16> { using type = uint4; };
 
-// Stores VEC values of TO at dst, which is aligned to min(16, VEC*sizeof(TO)),
-// with nontemporal stores (operator outputs are not re-read by the kernel).
+// Words of row pixels at any pixel's alignment: global accesses of 4 to 16
+// bytes need none on this device (a wave's row costs at most one more cache
+// line), so rows of odd pitch move as whole vectors too.
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned int u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned int u32_any __attribute__((aligned(1)));
+typedef unsigned short u16_any __attribute__((aligned(1)));
+
+// Stores VEC values of TO at dst: with nontemporal stores (operator outputs
+// are not re-read by the kernel) where dst is aligned to min(16, VEC *
+// sizeof(TO)), else with plain ones, so that the L2 joins the cache lines that
+// neighbouring tiles write in parts.
 template <typename TO, int VEC>
-__device__ __forceinline__ void store_vec(TO* dst, const TO (&v)[VEC]) {
+__device__ __forceinline__ void store_vec(TO* dst, const TO (&v)[VEC], bool aligned = true) {
   constexpr int BYTES = VEC * (int)sizeof(TO);
-  if constexpr (BYTES >= 16) {
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-    for (int k = 0; k < BYTES / 16; ++k) {
-      u32x4 w;
-      __builtin_memcpy(&w, reinterpret_cast<const char*>(v) + 16 * k, 16);
-      __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(dst) + k);
-    }
-  } else {
-    using W = typename std::conditional<
-        BYTES == 8, unsigned long long,
-        typename std::conditional<BYTES == 4, unsigned int,
-                                  typename std::conditional<BYTES == 2, unsigned short,
-                                                            unsigned char>::type>::type>::type;
-    W w;
-    __builtin_memcpy(&w, v, BYTES);
-    __builtin_nontemporal_store(w, reinterpret_cast<W*>(dst));
+  // (a macro: a template parameter would drop the types' alignment)
+#define HH_STORE_WORD(W, p, src)                                    \
+  {                                                                 \
+    W w;                                                            \
+    __builtin_memcpy(&w, src, sizeof(W));                           \
+    if (aligned) __builtin_nontemporal_store(w, (W*)(p));           \
+    else *(W*)(p) = w;                                              \
   }
+  if constexpr (BYTES >= 16) {
+#pragma unroll
+    for (int k = 0; k < BYTES / 16; ++k)
+      HH_STORE_WORD(u32x4_any, reinterpret_cast<char*>(dst) + 16 * k,
+                    reinterpret_cast<const char*>(v) + 16 * k)
+  } else if constexpr (BYTES == 8) {
+    HH_STORE_WORD(u32x2_any, dst, v)
+  } else if constexpr (BYTES == 4) {
+    HH_STORE_WORD(u32_any, dst, v)
+  } else if constexpr (BYTES == 2) {
+    HH_STORE_WORD(u16_any, dst, v)
+  } else {
+    static_assert(BYTES == 1, "pixel vector");
+    HH_STORE_WORD(unsigned char, dst, v)
+  }
+#undef HH_STORE_WORD
 }
 
 template <typename TI> __device__ __forceinline__ TI const_pixel(const Geom& g);
@@ -69,39 +85,42 @@ __device__ __forceinline__ void raw_region(const Geom& g, int& lx, int& hx, int&
   }
 }
 
+// Whether rows [iy0, iy0+lh) x columns [ix0, ix0+lw) all read raw pixels.
+__device__ __forceinline__ bool raw_tile(const Geom& g, int ix0, int iy0, int lw, int lh) {
+  int lx, hx, ly, hy;
+  raw_region(g, lx, hx, ly, hy);
+  return ix0 >= lx && ix0 + lw <= hx && iy0 >= ly && iy0 + lh <= hy;
+}
+
 // Stages rows [iy0, iy0+LH) x columns [ix0, ix0+NV*VEC) of the input into
 // tile (row pitch NV*VEC elements).
 template <typename TI, int VEC, int NV, int LH>
 __device__ __forceinline__ void stage_tile(TI* __restrict__ tile, const TI* __restrict__ in,
-                                           const Geom& g, int ix0, int iy0, int vec_ok) {
+                                           const Geom& g, int ix0, int iy0) {
   constexpr int LW = NV * VEC;
   const int tid = threadIdx.x;
-  int lx, hx, ly, hy;
-  raw_region(g, lx, hx, ly, hy);
-  const bool interior = vec_ok && ix0 >= lx && ix0 + LW <= hx && iy0 >= ly && iy0 + LH <= hy;
-  if (interior) {
+  if (raw_tile(g, ix0, iy0, LW, LH)) {
     // Every load of the thread is issued before the first LDS write, so all
-    // of them are in flight together.
-    constexpr int NL = (LH * NV + 255) / 256;
+    // of them are in flight together.  Threads past the last vector load it
+    // again: with the loads under a condition the staging array was placed in
+    // LDS and the loads waited for one by one, and the kernel read the
+    // workgroup size from the dispatch packet in host memory (7 us at the
+    // start of every launch).
+    constexpr int N = LH * NV, NL = (N + 255) / 256;
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     const TI* src = in + (long long)iy0 * g.in_stride + ix0;
-    uint4 w[NL];
+    u32x4 w[NL];
 #pragma unroll
     for (int k = 0; k < NL; ++k) {
-      const int i = tid + k * 256;
-      if (i < LH * NV) {
-        const int r = i / NV;
-        const int c = i - r * NV;
-        w[k] = *reinterpret_cast<const uint4*>(src + (long long)r * g.in_stride + c * VEC);
-      }
+      const int i = min(tid + k * 256, N - 1);
+      const int r = i / NV;
+      const int c = i - r * NV;
+      w[k] = *reinterpret_cast<const u32x4_any*>(src + (long long)r * g.in_stride + c * VEC);
     }
 #pragma unroll
     for (int k = 0; k < NL; ++k) {
       const int i = tid + k * 256;
-      if (i < LH * NV) {
-        const int r = i / NV;
-        const int c = i - r * NV;
-        *reinterpret_cast<uint4*>(tile + r * LW + c * VEC) = w[k];
-      }
+      if (i < N) *reinterpret_cast<u32x4*>(tile + i * VEC) = w[k];
     }
   } else {
     const bool cmode = g.boundary == HIPACC_BOUNDARY_CONSTANT;
@@ -155,8 +174,8 @@ __device__ __forceinline__ void store_row(TO* __restrict__ out, const Geom& g, i
     else
       vals[v] = convert_i<TO>((int32_t)acc[v], g.cvt, g.post_div);
   }
-  if (out_vec_ok && ox + VEC <= g.is_w) {
-    store_vec<TO, VEC>(dst, vals);
+  if (ox + VEC <= g.is_w) {
+    store_vec<TO, VEC>(dst, vals, out_vec_ok);
   } else {
 #pragma unroll
     for (int v = 0; v < VEC; ++v)

@@ -113,7 +113,7 @@ static int launch_ring(const LocalArgs& a0, int seg_rows, hipStream_t s) {
   if (strips * a.g.is_h * a.g.batch > (1ll << 31))
     return set_error(HIPACC_ERR_UNSUPPORTED, "ring kernel: %lld strip rows",
                      strips * a.g.is_h * a.g.batch);
-  const RingGeom rg = ring_geom(a.g, a.in_vec_ok, a.out_vec_ok, ring_edge_cost(K), 1, kRingV,
+  const RingGeom rg = ring_geom(a.g, 1, 1, ring_edge_cost(K), 1, kRingV,
                                 false, kRingChunk, seg_rows, ring_slots<K, FMA, WDEV>());
   hipLaunchKernelGGL((ring_kernel<K, FMA, WDEV, kRingChunk, kRingSets, ring_depth(K)>),
                      dim3(rg.items), dim3(256), 0, s, a, rg);
@@ -149,7 +149,7 @@ static int launch_ring_sep(const SepArgs& a0, int seg_rows, hipStream_t s) {
   if (strips * a.g.is_h * a.g.batch > (1ll << 31))
     return set_error(HIPACC_ERR_UNSUPPORTED, "ring_sep kernel: %lld strip rows",
                      strips * a.g.is_h * a.g.batch);
-  const RingGeom rg = ring_geom(a.g, a.in_vec_ok, a.out_vec_ok, 1.3f, HL, kRingV, false,
+  const RingGeom rg = ring_geom(a.g, 1, 1, 1.3f, HL, kRingV, false,
                                 sep_chunk<K>(), seg_rows, slots);
   hipLaunchKernelGGL((ring_sep_kernel<TI, TO, K, K, FMA, ISUM, sep_chunk<K>(), kRingSepSets>),
                      dim3(rg.items), dim3(256), 0, s, a, rg);

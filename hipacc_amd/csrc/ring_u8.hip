@@ -45,7 +45,13 @@ static int launch_ring8(const LocalArgs& a0, int seg_rows, hipStream_t s) {
 // The ring beats the streaming kernel once most strips are interior: at
 // 4096 columns (5 strips) 17 vs 20 us for a 3x3 Sobel u8 -> i16; at 1024
 // (2 edge strips) the streaming kernel's short segments win, 6.7 vs 9.6 us.
-bool ring8_pays(const LocalArgs& a) { return ceil_div(a.g.is_w, (64 - 2) * kRing8V) >= 4; }
+// Rows without 16-byte alignment would make every strip an edge strip of
+// per-pixel loads; the streaming kernel reads and writes them as whole words.
+bool ring8_pays(const LocalArgs& a) {
+  int in_ok = 0, out_ok = 0;
+  stream_align(a.g, kRing8V, in_ok, out_ok);
+  return in_ok && out_ok && ceil_div(a.g.is_w, (64 - 2) * kRing8V) >= 4;
+}
 
 int dispatch_ring8_local(const LocalArgs& a, int acc_is_float, int seg_rows, hipStream_t s) {
   const Geom& g = a.g;

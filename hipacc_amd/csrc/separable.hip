@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void separable_kernel(const SepArgs a) {
   const TI* in = static_cast<const TI*>(g.in) + (long long)blockIdx.z * g.in_plane;
   TO* out = static_cast<TO*>(g.out) + (long long)blockIdx.z * g.out_plane;
   const int iy0 = g.in_oy + ty0 - RY;
-  stage_tile<TI, VEC, NV, LH>(tile, in, g, g.in_ox + tx0 - HV * VEC, iy0, a.in_vec_ok);
+  stage_tile<TI, VEC, NV, LH>(tile, in, g, g.in_ox + tx0 - HV * VEC, iy0);
   __syncthreads();
 
   const int lane = threadIdx.x & 63;
