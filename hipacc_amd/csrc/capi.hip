@@ -927,9 +927,6 @@ int hipacc_hip_point(const hipacc_point_desc* d0, void* stream) {
   a.cvt = d->cvt;
   a.alpha = d->alpha;
   a.beta = d->beta;
-  const int e0 = dtype_bytes(d->in0.dtype), eo = dtype_bytes(o.dtype);
-  a.vec_ok = rows_aligned(d->in0, 4 * e0) && rows_aligned(o, 4 * eo) &&
-             (!binary || rows_aligned(d->in1, 4 * dtype_bytes(d->in1.dtype)));
   hipStream_t s = static_cast<hipStream_t>(stream);
   Timer tm(s);
   return tm.finish(launch_point(a, d->in0.dtype, binary ? d->in1.dtype : d->in0.dtype, o.dtype, s));

@@ -1,0 +1,55 @@
+"""Point operators in whole vectors: every tail length of a row, rows back to
+back and pitched, and the integer MAGNITUDE without divisions (quotients by
+any norm and square roots next to integers), bit for bit against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_binding as ob
+from gpu_util import empty_gpu, to_gpu, to_host
+from hipacc_amd import capi, operators as op
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tin,tout", [(np.uint8, np.uint8), (np.int16, np.uint8),
+                                      (np.uint8, np.float32), (np.float32, np.float32),
+                                      (np.float32, np.uint8), (np.int32, np.int16)])
+def test_point_tails(gpu, tin, tout):
+    kw = dict(src_dtype=ob.CODES[np.dtype(tin)], dst_dtype=ob.CODES[np.dtype(tout)])
+    for w in list(range(1, 18)) + [255, 4097]:
+        for h, pitch in ((1, 0), (3, 0), (3, w + 5)):
+            a, b = (ob.random_image((h, w), tin, s + w) for s in (1, 2))
+            for code, alpha in ((capi.POINT_AFFINE, 0.5), (capi.POINT_SUB, 1.0)):
+                two = code == capi.POINT_SUB
+                ref = np.zeros((h, w), tout)
+                ob.point(code, a, ref, b if two else None, alpha=alpha, beta=1.0)
+                buf = empty_gpu((h + 1, pitch or w), tout, fill=77)
+                dst = buf[:h, :w]
+                op.point(code, to_gpu(a, pitch), dst, to_gpu(b, pitch) if two else None,
+                         alpha=alpha, beta=1.0, **kw)
+                np.testing.assert_array_equal(to_host(dst, tout), ref)
+                dst[:] = 77
+                assert bool((buf == 77).all())
+
+
+@pytest.mark.parametrize("norm", [0, 1, 2, 3, 4, 7, 181, 255, 1000, 40000, -5])
+def test_magnitude_without_division(gpu, norm):
+    """All 16-bit values against others that make the sum of squares a square,
+    one more and one less; overflowing sums wrap."""
+    a = np.arange(-32768, 32768, dtype=np.int16).reshape(256, 256)
+    others = [np.zeros_like(a), a, np.full_like(a, 4), np.full_like(a, -1),
+              np.full_like(a, -32768), ob.random_image(a.shape, np.int16, norm & 255)]
+    for tin in (np.int16, np.uint16):
+        code = ob.CODES[np.dtype(tin)]
+        for b in others:
+            for tout, cvt in ((np.uint8, capi.CVT_TRUNC), (np.uint8, capi.CVT_ROUND),
+                              (np.int16, capi.CVT_TRUNC)):
+                ref = np.zeros(a.shape, tout)
+                ob.point(capi.POINT_MAGNITUDE, a.view(tin), ref, b.view(tin), alpha=float(norm),
+                         cvt=cvt)
+                dst = empty_gpu(a.shape, tout)
+                op.point(capi.POINT_MAGNITUDE, to_gpu(a.view(tin)), dst, to_gpu(b.view(tin)),
+                         alpha=float(norm), cvt=cvt, src_dtype=code,
+                         dst_dtype=ob.CODES[np.dtype(tout)])
+                np.testing.assert_array_equal(to_host(dst, tout), ref)
