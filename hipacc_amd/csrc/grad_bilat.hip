@@ -281,10 +281,10 @@ int launch_bilateral_grad(const BilatGradArgs& a0, float* dsigma, float sigma_r,
   a.tiles_x = ceil_div(a.w, 64);
   a.tiles_y = ceil_div(a.h, 16);
   a.ntiles = a.tiles_x * a.tiles_y * a.batch;
-  const int nblocks = a.ntiles < kGradBlocks ? a.ntiles : kGradBlocks;
+  int nblocks = a.ntiles < kGradBlocks ? a.ntiles : kGradBlocks;
   if (a.ksize > 15) return set_error(HIPACC_ERR_UNSUPPORTED, "bilateral_grad: ksize %d", a.ksize);
-  int st;
-  switch (a.ksize) {
+  int st = dispatch_bilat_pair_grad(a, &nblocks, s);
+  if (st == HIPACC_ERR_UNSUPPORTED) switch (a.ksize) {
     case 1: st = launch_bg<0>(a, nblocks, s); break;
     case 3: st = launch_bg<1>(a, nblocks, s); break;
     case 5: st = launch_bg<2>(a, nblocks, s); break;

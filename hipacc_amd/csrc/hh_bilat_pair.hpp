@@ -42,11 +42,11 @@ struct PairGeom {
 // Rows of a wave: the first wave's segment is shorter by the time of the rows
 // it walks above it (half of their pairs).  n minimises the blocks a CU gets x
 // the rows of a wave, with 1.5 rows for a segment's start and end.
-static inline PairGeom pair_geom(int w, int h, int batch, int r, int cus) {
+static inline PairGeom pair_geom(int w, int h, int batch, int r, int cus, int most = 1 << 30) {
   PairGeom best{};
   const int hl = (r + 3) / 4, s = 64 - 2 * hl;
   double bt = 0.0;
-  for (int n = r > 4 ? r : 4; n <= 128; ++n) {
+  for (int n = r > 4 ? r : 4; n <= 512; n += n < 128 ? 1 : 16) {
     PairGeom p;
     p.groups = ceil_div(w, 4);
     p.lb = p.groups + 2 * hl;
@@ -58,6 +58,7 @@ static inline PairGeom pair_geom(int w, int h, int batch, int r, int cus) {
     if (total >= (1ll << 30)) continue;
     p.total = (int)total;
     p.blocks = ceil_div(p.total, s);
+    if (p.blocks > most) continue;
     const int rounds = ceil_div(p.blocks, cus);
     // one or two waves per SIMD wait for their rows, the edge waves most
     const double t = (double)rounds * (n + 1.5) * (rounds == 1 ? 1.25 : rounds == 2 ? 1.08 : 1.0);

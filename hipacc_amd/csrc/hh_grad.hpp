@@ -185,5 +185,8 @@ struct BilatGradArgs {
 // and is added onto the band pixels of dX.
 int launch_bilateral_grad(const BilatGradArgs& a, float* dsigma, float sigma_r, float* ring,
                           hipStream_t s);
+// Its main kernel by pixel pairs (bilat_pair_grad.hip): HIPACC_ERR_UNSUPPORTED
+// where the tile kernel is to run; *nblocks: partials written.
+int dispatch_bilat_pair_grad(const BilatGradArgs& a, int* nblocks, hipStream_t s);
 
 }  // namespace hh
