@@ -217,12 +217,14 @@ HH_HD PyrRegion pyr_tile_region(int W, int H, int W1, int H1, int x0, int y0, in
 }
 
 // LDS capacity of a TW x TH tile kernel whose images have NN step
-// s = W / W1 <= SNUM / 4: the G[l+1] region (UW x UH) and the G[l] region
-// its blur taps span, at most ceil(s*(UW-1)) + 5 by ceil(s*(UH-1)) + 5.
+// s = W / W1 <= SNUM / 16: the G[l+1] region (UW x UH) and the G[l] region
+// its blur taps span, at most ceil(s*(UW-1)) + 5 by ceil(s*(UH-1)) + 5
+// (the width in whole 16-byte words: rows are staged four pixels at a time).
 template <int TW, int TH, int SNUM>
 struct PyrCap {
   static constexpr int UW = TW / 2 + 4, UH = TH / 2 + 4;
-  static constexpr int RW = (SNUM * (UW - 1) + 3) / 4 + 5, RH = (SNUM * (UH - 1) + 3) / 4 + 5;
+  static constexpr int RW = ((SNUM * (UW - 1) + 15) / 16 + 5 + 3) / 4 * 4;
+  static constexpr int RH = (SNUM * (UH - 1) + 15) / 16 + 5;
   HH_HD static bool fits(const PyrRegion& r) {
     return r.uw <= UW && r.uh <= UH && r.rw <= RW && r.rh <= RH;
   }

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "hh_pyramid.hpp"
+#include "hh_tile.hpp"
 
 namespace hh {
 
@@ -93,15 +94,22 @@ __device__ __forceinline__ float pyr_read(const float* g, int stride, int w, int
 // G[l+1] values the tile's LF reads and the ones it owns (columns x0/2..,
 // rows y0/2..) are computed -- the 5x5 convolution evaluated only at the NN
 // sample points -- the owned ones are stored, then L[l] = G[l] - LF(G[l+1]).
-// SNUM / 4 bounds the NN step s = W / W1 of every image in the work list:
-// 12 (s <= 3, any image) or 9 (s <= 2.25: images at least 9 pixels wide and
-// high at this level), which sizes the staged region.
+// SNUM / 16 bounds the NN step s = W / W1 of every image in the work list:
+// 48 (s <= 3, any image) or 33 (s <= 2 1/16: images at least 32 pixels wide
+// and high at this level), which sizes the staged region and with it the
+// blocks a CU holds (128 x 32 tiles: 5 at 33, where 36 gave 4).
+//
+// Bound by instruction issue and by how well the three phases of different
+// blocks overlap.  32 images of up to 4096 x 2160 (8 levels): 529 us with the
+// region staged pixel by pixel, the sample positions computed per G[l+1]
+// pixel and single-pixel stores; 390 us with four pixels per staging load,
+// per-lane columns in both phases and pixel pairs in the last one.
 template <int TW, int TH, int SNUM, bool FMA>
 __global__ __launch_bounds__(256) void pyramid_level_kernel(const PyrLevelArgs a) {
   using Cap = PyrCap<TW, TH, SNUM>;
   constexpr int UW = Cap::UW, UH = Cap::UH, RW = Cap::RW, RH = Cap::RH;
   __shared__ float g1s[UH * UW];
-  __shared__ float gls[RH * RW];
+  __shared__ __align__(16) float gls[RH * RW];
   const int l = a.level;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 
@@ -120,47 +128,49 @@ __global__ __launch_bounds__(256) void pyramid_level_kernel(const PyrLevelArgs a
     const int ux0 = rg.ux0, uy0 = rg.uy0, uw = rg.uw, uh = rg.uh;
     const int ox0 = rg.ox0, ox1 = rg.ox1, oy0 = rg.oy0, oy1 = rg.oy1;
     const int rx0 = rg.rx0, ry0 = rg.ry0, rw = rg.rw, rh = rg.rh;
-    const int rx1 = rx0 + rw - 1, ry1 = ry0 + rh - 1;
+    const int ry1 = ry0 + rh - 1;
     // The plan verified on the host (pyr_plan_tiles) that every tile of its
     // work lists fits; this guard only keeps LDS accesses in bounds.
     if (!Cap::fits(rg)) continue;
 
     __syncthreads();  // previous tile's LDS reads are done
-    // wave w stages rows w, w+4, ...; lane c the columns c, c+64, ...  Inside
-    // the image every load of the region is issued before the first LDS
-    // write, so the whole region is in flight at once.
-    if (rx0 >= 0 && ry0 >= 0 && rx1 < W && ry1 < H) {
-      constexpr int NR = (RH + 3) / 4, NC = (RW + 63) / 64;
-      float v[NR][NC];
+    // Four adjacent pixels of a region row per thread and turn; inside the
+    // image every load of the region is issued before the first LDS write,
+    // so the whole region is in flight at once.
+    const int nv = (rw + 3) >> 2, ni = nv * rh;
+    // i / nv and i / uw below as a multiply by the rounded-up reciprocal
+    // ceil(2^32 / n): exact for i < 2^32 / n; 1 has no 32-bit reciprocal and
+    // takes i itself
+    const unsigned rv = nv > 1 ? 0xffffffffu / (unsigned)nv + 1u : 0u;
+    constexpr int NL = (RW / 4 * RH + 255) / 256;
+    if (rx0 >= 0 && ry0 >= 0 && rx0 + 4 * nv <= W && ry1 < H) {
+      typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+      const float* src = G + (long long)ry0 * gs + rx0;
+      u32x4 v[NL];
+      int at[NL];
 #pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        const int r = wave + 4 * k;
-        const float* src = G + (long long)(ry0 + min(r, rh - 1)) * gs + rx0;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) v[k][c] = src[min(lane + 64 * c, rw - 1)];
+      for (int k = 0; k < NL; ++k) {
+        const int i = min((int)threadIdx.x + 256 * k, ni - 1);
+        const int r = nv > 1 ? (int)__umulhi((unsigned)i, rv) : i, c = (i - r * nv) * 4;
+        at[k] = r * RW + c;
+        v[k] = *reinterpret_cast<const u32x4_any*>(src + (long long)r * gs + c);
       }
 #pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        const int r = wave + 4 * k;
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-          if (r < rh && lane + 64 * c < rw) gls[r * RW + lane + 64 * c] = v[k][c];
-      }
+      for (int k = 0; k < NL; ++k)
+        if ((int)threadIdx.x + 256 * k < ni) *reinterpret_cast<u32x4*>(gls + at[k]) = v[k];
     } else {
-      for (int r = wave; r < rh; r += 4)
-        for (int c = lane; c < rw; c += 64)
-          gls[r * RW + c] = pyr_read(G, gs, W, H, a.boundary, rx0 + c, ry0 + r);
+      for (int i = threadIdx.x; i < ni; i += 256) {
+        const int r = nv > 1 ? (int)__umulhi((unsigned)i, rv) : i, c = (i - r * nv) * 4;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = pyr_read(G, gs, W, H, a.boundary, rx0 + c + e, ry0 + r);
+        *reinterpret_cast<float4*>(gls + r * RW + c) = make_float4(v[0], v[1], v[2], v[3]);
+      }
     }
     __syncthreads();
-    // i / uw as a multiply by the rounded-up reciprocal ceil(2^32 / uw):
-    // exact for i < 2^32 / uw (i < UW * UH here); uw == 1 has no 32-bit
-    // reciprocal and takes i itself
-    const unsigned recip = uw > 1 ? 0xffffffffu / (unsigned)uw + 1u : 0u;
-    for (int i = threadIdx.x; i < uw * uh; i += 256) {
-      const int yy = uw > 1 ? (int)__umulhi((unsigned)i, recip) : i, xx = i - yy * uw;
-      const int xu = ux0 + xx, yu = uy0 + yy;
-      const int nx = (int)interp_map(sd, xu) - 2 - rx0, ny = (int)interp_map(td, yu) - 2 - ry0;
-      const float* src = gls + ny * RW + nx;
+    // G[l+1] pixel (xx, yy) of the region from the G[l] taps at src
+    auto blur = [&](const float* src, int xx, int yy) {
       float acc = 0.0f;
 #pragma unroll
       for (int ty = 0; ty < 5; ++ty)
@@ -174,42 +184,74 @@ __global__ __launch_bounds__(256) void pyramid_level_kernel(const PyrLevelArgs a
             acc = madd<FMA>(wv, v, acc);
         }
       g1s[yy * UW + xx] = acc;
+      const int xu = ux0 + xx, yu = uy0 + yy;
       if (xu >= ox0 && xu <= ox1 && yu >= oy0 && yu <= oy1)
         G1[(long long)yu * g1st + xu] = acc;
+    };
+    // the region's first columns one per lane (a wave walks rows wave,
+    // wave + 4, ...), the rest of a wide tile's region and a narrow tile's
+    // one pixel per thread
+    constexpr int XC = TW >= 128 ? 64 : 0;
+    if (XC && lane < uw) {
+      const int nx = (int)interp_map(sd, ux0 + lane) - 2 - rx0;
+      for (int yy = wave; yy < uh; yy += 4) {
+        const int ny = (int)interp_map(td, uy0 + yy) - 2 - ry0;
+        blur(gls + ny * RW + nx, lane, yy);
+      }
+    }
+    const int xr = uw - XC;
+    if (xr > 0) {
+      const unsigned recip = xr > 1 ? 0xffffffffu / (unsigned)xr + 1u : 0u;
+      for (int i = threadIdx.x; i < xr * uh; i += 256) {
+        const int yy = xr > 1 ? (int)__umulhi((unsigned)i, recip) : i, xx = XC + i - yy * xr;
+        const int nx = (int)interp_map(sd, ux0 + xx) - 2 - rx0;
+        const int ny = (int)interp_map(td, uy0 + yy) - 2 - ry0;
+        blur(gls + ny * RW + nx, xx, yy);
+      }
     }
     __syncthreads();
 
-    // a lane keeps the columns lane, lane+64, ... (their LF column weights
-    // are computed once) and walks the rows wave, wave+4, ... (the row's LF
-    // weights computed once for all its columns)
+    // a lane keeps NCX adjacent columns (their LF column weights are computed
+    // once) and walks the rows wave, wave+4, ... (the row's LF weights
+    // computed once for all its columns)
     constexpr int NCX = TW / 64;
     int xa[NCX], xb[NCX];
     float fx[NCX];
+    const int xl = x0 + NCX * lane;
 #pragma unroll
     for (int cx = 0; cx < NCX; ++cx) {
-      const int x = x0 + lane + 64 * cx;
       int xi;
-      interp_lf(interp_map(su, x), xi, fx[cx]);
+      interp_lf(interp_map(su, min(xl + cx, W - 1)), xi, fx[cx]);
       xa[cx] = xi - ux0;
       xb[cx] = min(xi + 1, W1 - 1) - ux0;
     }
     const int rows = min(TH, H - y0);
-    for (int r = wave; r < rows; r += 4) {
-      const int y = y0 + r;
-      int yi;
-      float fy;
-      interp_lf(interp_map(sv, y), yi, fy);
-      const int ya = (yi - uy0) * UW, yb = (min(yi + 1, H1 - 1) - uy0) * UW;
-      const int grow = (y - ry0) * RW - rx0;
-      float* lrow = L + (long long)y * ls;
+    if (xl < W) {
+      for (int r = wave; r < rows; r += 4) {
+        const int y = y0 + r;
+        int yi;
+        float fy;
+        interp_lf(interp_map(sv, y), yi, fy);
+        const int ya = (yi - uy0) * UW, yb = (min(yi + 1, H1 - 1) - uy0) * UW;
+        const float* grow = gls + (y - ry0) * RW - rx0 + xl;
+        float* lrow = L + (long long)y * ls + xl;
+        float v[NCX];
 #pragma unroll
-      for (int cx = 0; cx < NCX; ++cx) {
-        const int x = x0 + lane + 64 * cx;
-        if (x < W) {
-          const float lf = interp_bilinear(fx[cx], fy, g1s[ya + xa[cx]], g1s[ya + xb[cx]],
-                                           g1s[yb + xa[cx]], g1s[yb + xb[cx]]);
-          // L[l] is not read again here: non-temporal stores
-          __builtin_nontemporal_store(gls[grow + x] - lf, lrow + x);
+        for (int cx = 0; cx < NCX; ++cx)
+          v[cx] = grow[cx] - interp_bilinear(fx[cx], fy, g1s[ya + xa[cx]], g1s[ya + xb[cx]],
+                                             g1s[yb + xa[cx]], g1s[yb + xb[cx]]);
+        // L[l] is not read again here: non-temporal stores
+        if constexpr (NCX == 2) {
+          typedef float pyr_f2 __attribute__((ext_vector_type(2), aligned(4)));
+          if (xl + 1 < W) {
+            const pyr_f2 q = {v[0], v[1]};
+            __builtin_nontemporal_store(q, reinterpret_cast<pyr_f2*>(lrow));
+          } else {
+            __builtin_nontemporal_store(v[0], lrow);
+          }
+        } else {
+          static_assert(NCX == 1, "tile width");
+          __builtin_nontemporal_store(v[0], lrow);
         }
       }
     }
@@ -235,6 +277,7 @@ struct hipacc_pyramid_plan {
 namespace hh {
 
 constexpr int kPyrWideMin = 512;    // wide tiles of a level worth a wide launch
+constexpr int kPyrWideSize = 32;    // pixels of an image side whose NN step is <= 2 1/16
 
 template <int TW, int TH, int SNUM, bool FMA>
 static int launch_level_t(const PyrLevelArgs& a, hipStream_t s) {
@@ -246,10 +289,10 @@ static int launch_level_t(const PyrLevelArgs& a, hipStream_t s) {
 
 template <bool FMA>
 static int launch_level(const PyrLevelArgs& a, bool wide, int tile_rows, hipStream_t s) {
-  if (wide) return launch_level_t<128, 32, 9, FMA>(a, s);
-  return tile_rows == 8    ? launch_level_t<64, 8, 12, FMA>(a, s)
-         : tile_rows == 32 ? launch_level_t<64, 32, 12, FMA>(a, s)
-                           : launch_level_t<64, 16, 12, FMA>(a, s);
+  if (wide) return launch_level_t<128, 32, 33, FMA>(a, s);
+  return tile_rows == 8    ? launch_level_t<64, 8, 48, FMA>(a, s)
+         : tile_rows == 32 ? launch_level_t<64, 32, 48, FMA>(a, s)
+                           : launch_level_t<64, 16, 48, FMA>(a, s);
 }
 
 static int plan_launches(hipacc_pyramid_plan* p, hipStream_t s) {
@@ -273,8 +316,8 @@ static int plan_launches(hipacc_pyramid_plan* p, hipStream_t s) {
   return HIPACC_OK;
 }
 
-// Work lists of every level: images at least 9 x 9 at a level (NN step
-// <= 2.25) may take wide 128 x 32 tiles; a level takes them when there are
+// Work lists of every level: images at least 32 x 32 at a level (NN step
+// <= 2 1/16) may take wide 128 x 32 tiles; a level takes them when there are
 // at least kPyrWideMin (they fill the device several times over), and the
 // smaller images of that level, or every image of a smaller level, take
 // narrow 64 x tile_rows tiles.  Every tile's staged regions are computed with
@@ -295,7 +338,7 @@ static int pyr_plan_tiles(const int* w0, const int* h0, int n, int levels, int t
         return set_error(HIPACC_ERR_INVALID_ARG, "pyramid: image %d too small for %d levels", i,
                          levels);
       if (l + 1 < levels) {
-        if (w >= 9 && h >= 9)
+        if (w >= kPyrWideSize && h >= kPyrWideSize)
           for (int y0 = 0; y0 < h; y0 += 32)
             for (int x0 = 0; x0 < w; x0 += 128) wlists[l].push_back(PyrTile{i, x0, y0});
         for (int y0 = 0; y0 < h; y0 += tile_rows)
@@ -310,7 +353,7 @@ static int pyr_plan_tiles(const int* w0, const int* h0, int n, int levels, int t
   for (int l = 0; l + 1 < levels; ++l) {
     if ((int)wlists[l].size() >= kPyrWideMin) {
       for (const PyrTile& t : nlists[l])
-        if (lw(t.img, l) < 9 || lh(t.img, l) < 9) lists[l].push_back(t);
+        if (lw(t.img, l) < kPyrWideSize || lh(t.img, l) < kPyrWideSize) lists[l].push_back(t);
     } else {
       wlists[l].clear();
       lists[l] = nlists[l];
@@ -320,10 +363,10 @@ static int pyr_plan_tiles(const int* w0, const int* h0, int n, int levels, int t
         const int Wl = lw(t.img, l), Hl = lh(t.img, l);
         const int TW = wide ? 128 : 64, TH = wide ? 32 : tile_rows;
         const PyrRegion r = pyr_tile_region(Wl, Hl, Wl / 2, Hl / 2, t.x0, t.y0, TW, TH);
-        const bool ok = wide ? PyrCap<128, 32, 9>::fits(r)
-                        : tile_rows == 8  ? PyrCap<64, 8, 12>::fits(r)
-                        : tile_rows == 32 ? PyrCap<64, 32, 12>::fits(r)
-                                          : PyrCap<64, 16, 12>::fits(r);
+        const bool ok = wide ? PyrCap<128, 32, 33>::fits(r)
+                        : tile_rows == 8  ? PyrCap<64, 8, 48>::fits(r)
+                        : tile_rows == 32 ? PyrCap<64, 32, 48>::fits(r)
+                                          : PyrCap<64, 16, 48>::fits(r);
         if (!ok)
           return set_error(HIPACC_ERR_INVALID_ARG,
                            "pyramid: image %d level %d tile (%d, %d) stages %dx%d / %dx%d "
