@@ -40,13 +40,18 @@ typedef unsigned short u16_any __attribute__((aligned(1)));
 template <typename TO, int VEC>
 __device__ __forceinline__ void store_vec(TO* dst, const TO (&v)[VEC], bool aligned = true) {
   constexpr int BYTES = VEC * (int)sizeof(TO);
-  // (a macro: a template parameter would drop the types' alignment)
+  // (a macro: a template parameter would drop the types' alignment; the empty
+  // asm keeps the compiler from joining both stores into a plain one)
 #define HH_STORE_WORD(W, p, src)                                    \
   {                                                                 \
     W w;                                                            \
     __builtin_memcpy(&w, src, sizeof(W));                           \
-    if (aligned) __builtin_nontemporal_store(w, (W*)(p));           \
-    else *(W*)(p) = w;                                              \
+    if (aligned) {                                                  \
+      __builtin_nontemporal_store(w, (W*)(p));                      \
+    } else {                                                        \
+      *(W*)(p) = w;                                                 \
+      asm volatile("" ::: "memory");                                \
+    }                                                               \
   }
   if constexpr (BYTES >= 16) {
 #pragma unroll
