@@ -320,21 +320,21 @@ __device__ __forceinline__ void points_vec(const FusedArgs& a, int from, int to,
                                            FastV<T> (&v)[N], XY&& xy, int b) {
   for (int k = from; k < to; ++k) {
     const FusedPoint& s = a.pt[k];
+    if (!s.in1.data) {
+      // one-input operators (the others always have a second input) without
+      // the decode and the zeros of one (Mixed chain at 4096^2: 80.3 -> 78.2 us)
+      if (s.op == HIPACC_POINT_AFFINE) point_op_vec<T, HIPACC_POINT_AFFINE, N>(s, v, v);
+      else point_op_vec<T, HIPACC_POINT_COPY, N>(s, v, v);
+      continue;
+    }
     FastV<T> u[N];
-    if (s.in1.data) {
-      const T* p = static_cast<const T*>(s.in1.data) + (long long)b * s.in1.plane;
+    const T* p = static_cast<const T*>(s.in1.data) + (long long)b * s.in1.plane;
 #pragma unroll
-      for (int e = 0; e < N; ++e) {
-        const int2 q = xy(e);
-        u[e] = (FastV<T>)p[(long long)(s.in1.oy + q.y) * s.in1.stride + s.in1.ox + q.x];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < N; ++e) u[e] = 0;
+    for (int e = 0; e < N; ++e) {
+      const int2 q = xy(e);
+      u[e] = (FastV<T>)p[(long long)(s.in1.oy + q.y) * s.in1.stride + s.in1.ox + q.x];
     }
     switch (s.op) {
-      case HIPACC_POINT_COPY: point_op_vec<T, HIPACC_POINT_COPY, N>(s, v, u); break;
-      case HIPACC_POINT_AFFINE: point_op_vec<T, HIPACC_POINT_AFFINE, N>(s, v, u); break;
       case HIPACC_POINT_ADD: point_op_vec<T, HIPACC_POINT_ADD, N>(s, v, u); break;
       case HIPACC_POINT_SUB: point_op_vec<T, HIPACC_POINT_SUB, N>(s, v, u); break;
       case HIPACC_POINT_MUL: point_op_vec<T, HIPACC_POINT_MUL, N>(s, v, u); break;
