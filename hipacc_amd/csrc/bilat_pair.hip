@@ -66,7 +66,12 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
   };
 
   float ref = 0.0f;                        // pixels are scaled about this value
-  const float sc = __builtin_sqrtf(-a.k2), isc = 1.0f / sc;
+  // Factors as sums of two floats: a factor's own rounding would shift sigma
+  // for every pixel alike, where a product rounded once is off at random (the
+  // gradient for sigma is a sum that cancels and shows the difference).
+  const float sc = (float)a.scale, scl = (float)(a.scale - (double)sc);
+  const double inv = 1.0 / a.scale;
+  const float isc = (float)inv, iscl = (float)(inv - (double)isc);
   const float s0 = __builtin_amdgcn_exp2f(a.lsp[R * K + R]);
   // x, den, num: scaled pixels of row y and their sums (without the centre tap)
   auto finish = [&](int y, const float (&x)[V], const float (&den)[V], const float (&num)[V]) {
@@ -78,7 +83,8 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
       // with a centre weight the sum is no denormal and the reciprocal's last
       // bit only scales the correction SUM s d / SUM s
       const float q = s0 > 1e-30f ? num[e] * __builtin_amdgcn_rcpf(n[e]) : num[e] / n[e];
-      r[e] = __builtin_fmaf(x[e] + q, isc, ref);
+      const float xq = x[e] + q;
+      r[e] = __builtin_fmaf(xq, isc, __builtin_fmaf(xq, iscl, ref));
     }
     float* dst = static_cast<float*>(g.out) + (long long)pl.b * g.out_plane +
                  (long long)(g.out_oy + y) * g.out_stride + g.out_ox + pl.x;
@@ -106,7 +112,10 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
   float den[R + 1][V], num[R + 1][V];      // sums of rows y .. y + R
   auto scaled = [&](const float (&v)[V], float (&x)[V]) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) x[e] = (v[e] - ref) * sc;
+    for (int e = 0; e < V; ++e) {
+      const float d = v[e] - ref;
+      x[e] = __builtin_fmaf(d, sc, d * scl);
+    }
   };
   {
     float v[R + 1][V];

@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
   constexpr int V = 4, K = 2 * R + 1, HL = (R + V - 1) / V, NW = V + 2 * R;
   constexpr float kKappa = 1.38629436111989061883f;   // 2 ln 2
   __shared__ __align__(16) float4 part[3][R][3][64];  // first R rows of waves 1..3: N, S2, S3
-  __shared__ float red[4];
+  __shared__ double red[4];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const PairLane pl = pair_lane<HL>(pg, lane, 3 * pg.n + pg.n0);
@@ -88,8 +88,9 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
     }
   };
 
-  const float sc = __builtin_sqrtf(-a.k2);
+  const float sc = (float)a.scale, scl = (float)(a.scale - (double)sc);   // as in bilat_pair_kernel
   const float s0 = a.sp[R * K + R], c2 = 2.0f * a.c, bsc = kKappa * sc;
+  const double zsc = a.scale / (double)bsc;   // b * zsc = a z sqrt(c log2 e)
   float ref = 0.0f;
   float xr[R + 1][V], ar[R + 1][V], br[R + 1][V];      // rows y .. y + R
   float nn[R + 1][V], s2[R + 1][V], s3[R + 1][V];      // their sums
@@ -100,7 +101,8 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       const float av = r.g[e] / r.d[e], z = r.x[e] - r.y[e];
-      xr[k][e] = (r.x[e] - ref) * sc;
+      const float xd = r.x[e] - ref;
+      xr[k][e] = __builtin_fmaf(xd, sc, xd * scl);
       ar[k][e] = av;
       br[k][e] = av * (z * bsc);
       nn[k][e] = own ? __builtin_fmaf(-c2 * z * z, r.g[e], av * s0) : 0.0f;
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
       s3[k][e] = 0.0f;
     }
   };
-  float dc = 0.0f;
+  double dc = 0.0;   // the two terms cancel largely, and the pixels' sums too
   auto finish = [&](int y, const float (&av)[V], const float (&bv)[V], const float (&n)[V],
                     const float (&t2)[V], const float (&t3)[V]) {
     if (!pl.store || y >= a.h) return;
@@ -117,8 +119,7 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
     for (int e = 0; e < V; ++e) {
       v[e] = __builtin_fmaf(kKappa * av[e], t2[e], n[e]);
       // a and b are 0 for the columns beside the image
-      dc = __builtin_fmaf(av[e], t3[e], dc);
-      dc = __builtin_fmaf(bv[e] * (1.0f / kKappa), t2[e], dc);
+      dc += (double)av[e] * (double)t3[e] + zsc * ((double)bv[e] * (double)t2[e]);
     }
     float* dst = a.gx + (long long)pl.b * a.gx_plane + (long long)y * a.gx_stride + pl.x;
     if (pl.x + V <= a.w) {
@@ -246,12 +247,14 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
       finish(y, ar[k], br[k], n, t2, t3);
     }
   }
-  dc = wave_sum(dc);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) dc += __shfl_xor(dc, off, 64);
   if (lane == 0) red[wave] = dc;
   __syncthreads();
   if (threadIdx.x == 0) {
-    const float isc = 1.0f / sc;
-    a.partials[blockIdx.x] = -((((red[0] + red[1]) + red[2]) + red[3]) * isc) * isc * isc;
+    const double isc = 1.0 / a.scale;
+    a.partials[blockIdx.x] =
+        (float)(-(((red[0] + red[1]) + red[2]) + red[3]) * (isc * isc * isc));
   }
 }
 

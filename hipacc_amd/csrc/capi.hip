@@ -485,6 +485,12 @@ static int prep_separable(const hipacc_separable_desc* d, SepArgs& a, int& accf)
   return HIPACC_OK;
 }
 
+// sqrt(log2(e) / (2 sigma^2)): pixel differences times it, squared, are the
+// range weight's negative exponent to base 2.
+static double bilat_scale(float sigma_r) {
+  return std::sqrt(0.5 * 1.44269504088896340736) / (double)sigma_r;
+}
+
 static int run_local(const hipacc_local_desc* d, int variant, int param, hipStream_t s) {
   LocalArgs a;
   SepArgs sa;
@@ -1053,6 +1059,7 @@ int hipacc_hip_bilateral(const hipacc_bilateral_desc* d, void* stream) {
     }
   const float c_r = 0.5f / (d->sigma_r * d->sigma_r);
   a.k2 = -c_r * 1.44269504088896340736f;
+  a.scale = bilat_scale(d->sigma_r);
   a.in_vec_ok = d->in.dtype == HIPACC_F32 && rows_aligned(d->in, 16) && (d->in.offset_x % 4) == 0;
   a.out_vec_ok = rows_aligned(d->out, 4 * dtype_bytes(d->out.dtype));
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1300,6 +1307,7 @@ int hipacc_hip_bilateral_train(const hipacc_bilateral_grad_desc* d, void* stream
   for (int t = 0; t < d->ksize * d->ksize; ++t) a.lsp[t] = sp[t] > 0.0f ? std::log2(sp[t]) : -INFINITY;
   const float c_r = 0.5f / (d->sigma_r * d->sigma_r);
   a.k2 = -c_r * 1.44269504088896340736f;
+  a.scale = bilat_scale(d->sigma_r);
   a.in_vec_ok = rows_aligned(d->in, 16);
   a.out_vec_ok = rows_aligned(d->out, 16);
   a.norm = static_cast<float*>(d->norm.data);
@@ -1365,6 +1373,7 @@ int hipacc_hip_bilateral_grad(const hipacc_bilateral_grad_desc* d, void* stream)
   a.cval = (float)d->const_val;
   a.c = 0.5f / (d->sigma_r * d->sigma_r);
   a.k2 = -a.c * 1.44269504088896340736f;
+  a.scale = bilat_scale(d->sigma_r);
   a.vec_ok = rows_aligned(d->in, 16) && rows_aligned(d->out, 16) && rows_aligned(d->norm, 16) &&
              rows_aligned(d->grad_out, 16) && (!dx || rows_aligned(d->grad_in, 16));
   const size_t total = hipacc_hip_bilateral_grad_workspace_bytes(d);

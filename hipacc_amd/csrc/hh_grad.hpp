@@ -171,6 +171,7 @@ struct BilatGradArgs {
   float cval;
   float c;             // 0.5 / sigma_r^2
   float k2;            // -c * log2(e)
+  double scale;        // sqrt(c * log2(e)) of the float sigma_r
   float sp[kMaxTaps];  // spatial weights
   float lsp[kMaxTaps]; // log2 of the spatial weights
   int sym;             // sp is point-symmetric

@@ -166,6 +166,7 @@ struct BilatArgs {
   int ksize;
   int in_vec_ok, out_vec_ok;
   float k2;                 // -c_r * log2(e)
+  double scale;             // sqrt(c_r * log2(e)) of the float sigma_r
   float lsp[kMaxTaps];      // log2(spatial)
   float* norm;              // F32 out only: per-pixel SUM of weights, or NULL
   long long norm_plane;
