@@ -64,8 +64,15 @@ def view(t: torch.Tensor, window: Window = None, dtype: Optional[int] = None) ->
     return v
 
 
+# The raw handle of torch's current stream on the current device, without the
+# Stream object of torch.cuda.current_stream() (2 us of a small operator's
+# 6 us call).
+_device = torch._C._cuda_getDevice
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 class Call:
