@@ -975,7 +975,6 @@ int hipacc_hip_reduce(const hipacc_view* img, int32_t reduce, int32_t acc_dtype,
   a.w = img->width;
   a.h = img->height;
   a.mode = reduce;
-  a.vec_ok = rows_aligned(*img, 16);
   a.result = result_dev;
   a.partials = static_cast<unsigned long long*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1019,7 +1018,6 @@ int hipacc_hip_histogram(const hipacc_view* img, int32_t num_bins, float scale, 
   a.h = img->height;
   a.nbins = num_bins;
   a.scale = scale;
-  a.vec_ok = rows_aligned(*img, 16);
   a.bins = bins_dev;
   hipStream_t s = static_cast<hipStream_t>(stream);
   void* ws = nullptr;

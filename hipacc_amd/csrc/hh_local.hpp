@@ -135,7 +135,6 @@ struct ReduceArgs {
   const void* in;
   int stride, ox, oy, w, h;
   int mode;
-  int vec_ok;
   void* result;
   unsigned long long* partials;   // kRedBlocks entries
 };
@@ -147,7 +146,6 @@ struct HistArgs {
   int stride, ox, oy, w, h;
   int nbins;
   float scale;
-  int vec_ok;
   uint32_t* bins;
   uint32_t* partials;   // [blocks][nbins] per-block histograms (workspace)
 };

@@ -2,8 +2,9 @@
 // small utility kernels (fill, synthetic pixels, window copy).
 //
 // Reduction: a fixed grid of blocks walks the window's rows (block b takes
-// rows b, b+G, ...; threads stride along the row with 16-byte loads when the
-// row is aligned, keeping the loads of 4 rows in flight together).  Each wave folds its 64 lanes with cross-lane shuffles,
+// rows b, b+G, ...; threads stride along the row with 16-byte loads at any
+// alignment, keeping the loads of 4 rows in flight together; rows back to
+// back are one sweep).  Each wave folds its 64 lanes with cross-lane shuffles,
 // one LDS level folds the 4 waves, and block partials go to the workspace.
 // A second one-block kernel folds the partials in a fixed order and writes
 // the result, so the result does not depend on scheduling.  (A last-block
@@ -12,6 +13,8 @@
 #include "hh_tile.hpp"
 
 namespace hh {
+
+typedef unsigned int red_u4 __attribute__((ext_vector_type(4)));
 
 template <typename A> __device__ __forceinline__ A red_identity(int mode);
 template <> __device__ __forceinline__ float red_identity<float>(int mode) {
@@ -77,15 +80,16 @@ __global__ __launch_bounds__(256) void reduce_kernel(const ReduceArgs a) {
   const int G = gridDim.x;
   A acc = red_identity<A>(mode);
   const T* base = static_cast<const T*>(a.in) + (long long)a.oy * a.stride + a.ox;
-  if (a.vec_ok && a.stride == a.w) {
+  if (a.stride == a.w) {
     // rows back to back: one grid-stride sweep, so that the whole grid reads
-    // one contiguous stretch of memory at a time
+    // one contiguous stretch of memory at a time, in 16-byte words whatever
+    // the base's alignment
     const long long nv = (long long)a.h * a.w / VEC;
     const long long st = (long long)G * 256;
-    const uint4* v = reinterpret_cast<const uint4*>(base);
+    const u32x4_any* v = reinterpret_cast<const u32x4_any*>(base);
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     for (; i + (U - 1) * st < nv; i += U * st) {
-      uint4 w[U];
+      red_u4 w[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) w[u] = v[i + u * st];
 #pragma unroll
@@ -97,7 +101,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(const ReduceArgs a) {
       }
     }
     for (; i < nv; i += st) {
-      const uint4 w = v[i];
+      const red_u4 w = v[i];
       T t[VEC];
       __builtin_memcpy(t, &w, 16);
 #pragma unroll
@@ -110,37 +114,28 @@ __global__ __launch_bounds__(256) void reduce_kernel(const ReduceArgs a) {
   // block b folds rows b, b+G, ...; a thread loads the same vector of U of
   // its block's rows at once
   for (int y0 = blockIdx.x; y0 < a.h; y0 += U * G) {
-    if (a.vec_ok) {
-      const int nv = a.w / VEC;
-      for (int i = threadIdx.x; i < nv; i += 256) {
-        uint4 w[U];
+    const int nv = a.w / VEC;
+    for (int i = threadIdx.x; i < nv; i += 256) {
+      red_u4 w[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int y = y0 + u * G;
-          if (y < a.h) w[u] = reinterpret_cast<const uint4*>(base + (long long)y * a.stride)[i];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (y0 + u * G >= a.h) break;
-          T t[VEC];
-          __builtin_memcpy(t, &w[u], 16);
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) acc = red_op<A>(mode, acc, (A)t[k]);
-        }
-      }
       for (int u = 0; u < U; ++u) {
         const int y = y0 + u * G;
-        if (y >= a.h) break;
-        const T* row = base + (long long)y * a.stride;
-        for (int x = nv * VEC + threadIdx.x; x < a.w; x += 256) acc = red_op<A>(mode, acc, (A)row[x]);
+        if (y < a.h) w[u] = reinterpret_cast<const u32x4_any*>(base + (long long)y * a.stride)[i];
       }
-    } else {
+#pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int y = y0 + u * G;
-        if (y >= a.h) break;
-        const T* row = base + (long long)y * a.stride;
-        for (int x = threadIdx.x; x < a.w; x += 256) acc = red_op<A>(mode, acc, (A)row[x]);
+        if (y0 + u * G >= a.h) break;
+        T t[VEC];
+        __builtin_memcpy(t, &w[u], 16);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc = red_op<A>(mode, acc, (A)t[k]);
       }
+    }
+    for (int u = 0; u < U; ++u) {
+      const int y = y0 + u * G;
+      if (y >= a.h) break;
+      const T* row = base + (long long)y * a.stride;
+      for (int x = nv * VEC + threadIdx.x; x < a.w; x += 256) acc = red_op<A>(mode, acc, (A)row[x]);
     }
   }
   acc = block_fold<A>(mode, acc, sm);
@@ -171,8 +166,8 @@ template <typename T, typename A>
 static int launch_reduce_t(const ReduceArgs& a, hipStream_t s) {
   const long long n = (long long)a.w * a.h;
   const int flat_blocks = (int)((n + 4095) / 4096 < kRedBlocks ? (n + 4095) / 4096 : kRedBlocks);
-  const int blocks = (a.vec_ok && a.stride == a.w) ? (flat_blocks > 0 ? flat_blocks : 1)
-                                                   : (a.h < kRedBlocks ? a.h : kRedBlocks);
+  const int blocks = a.stride == a.w ? (flat_blocks > 0 ? flat_blocks : 1)
+                                     : (a.h < kRedBlocks ? a.h : kRedBlocks);
 #define HH_RED(M)                                                                         \
   hipLaunchKernelGGL((reduce_kernel<T, A, M>), dim3(blocks), dim3(256), 0, s, a);         \
   hipLaunchKernelGGL((reduce_final_kernel<A, M>), dim3(1), dim3(256), 0, s, a.partials, blocks, \
@@ -246,13 +241,13 @@ __global__ __launch_bounds__(kHistThreads) void hist_partial_kernel(const HistAr
       if (b >= 0 && b < a.nbins) atomicAdd(mine + b * NC, 1u);
     }
   };
-  auto count = [&](const uint4& w) {
+  auto count = [&](const red_u4& w) {
     T t[VEC];
     __builtin_memcpy(t, &w, 16);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) count1(t[k]);
   };
-  if (a.vec_ok && a.stride == a.w) {
+  if (a.stride == a.w) {
     // Rows back to back: block b takes the contiguous vectors
     // [b*nv/G, (b+1)*nv/G).  Each thread keeps the loads of its next U
     // vectors in flight while it counts the current U.
@@ -261,14 +256,14 @@ __global__ __launch_bounds__(kHistThreads) void hist_partial_kernel(const HistAr
     const long long n = (long long)a.h * a.w;
     const long long nv = n / VEC;
     const long long b0 = nv * blockIdx.x / gridDim.x, b1 = nv * (blockIdx.x + 1) / gridDim.x;
-    const uint4* v = reinterpret_cast<const uint4*>(base);
+    const u32x4_any* v = reinterpret_cast<const u32x4_any*>(base);
     long long i = b0 + threadIdx.x;
     if (i + (U - 1) * NT < b1) {
-      uint4 cur[U];
+      red_u4 cur[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) cur[u] = v[i + u * NT];
       for (i += U * NT; i + (U - 1) * NT < b1; i += U * NT) {
-        uint4 nxt[U];
+        red_u4 nxt[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) nxt[u] = v[i + u * NT];
 #pragma unroll
@@ -279,19 +274,21 @@ __global__ __launch_bounds__(kHistThreads) void hist_partial_kernel(const HistAr
 #pragma unroll
       for (int u = 0; u < U; ++u) count(cur[u]);
     }
-    for (; i < b1; i += NT) count(v[i]);
+    for (; i < b1; i += NT) {
+      const red_u4 w = v[i];
+      count(w);
+    }
     if (blockIdx.x == gridDim.x - 1)
       for (long long x = nv * VEC + threadIdx.x; x < n; x += NT) count1(base[x]);
   } else {
     for (int y = blockIdx.x; y < a.h; y += gridDim.x) {
       const T* row = static_cast<const T*>(a.in) + (long long)(a.oy + y) * a.stride + a.ox;
-      int start = 0;
-      if (a.vec_ok) {
-        const int nv = a.w / VEC;
-        for (int i = threadIdx.x; i < nv; i += NT) count(reinterpret_cast<const uint4*>(row)[i]);
-        start = nv * VEC;
+      const int nv = a.w / VEC;
+      for (int i = threadIdx.x; i < nv; i += NT) {
+        const red_u4 w = reinterpret_cast<const u32x4_any*>(row)[i];
+        count(w);
       }
-      for (int x = start + threadIdx.x; x < a.w; x += NT) count1(row[x]);
+      for (int x = nv * VEC + threadIdx.x; x < a.w; x += NT) count1(row[x]);
     }
   }
   __syncthreads();
@@ -334,7 +331,7 @@ int launch_histogram(const HistArgs& a, int dt, hipStream_t s) {
   // 9.9 us for both launches; 16, 32 and 128 KiB: 11.2-11.4 us), at most 512
   // blocks; other windows: one block per row.  blocks * nbins entries must
   // fit the partials workspace.
-  const bool flat = a.vec_ok && a.stride == a.w;
+  const bool flat = a.stride == a.w;
   const long long chunk = 64 * 1024;
   const long long want = flat ? (n * eb + chunk - 1) / chunk : a.h;
   long long blocks = want < 512 ? want : 512;

@@ -101,3 +101,26 @@ def test_bilateral_unaligned(gpu, mode):
         op.bilateral(pitched, ref, 7, 2.0, sr, boundary=mode, const_val=0.5, cvt=cvt)
         _run(op.bilateral, src, dtype, 3, mode, to_host(ref, dtype), ksize=7, sigma_d=2.0,
              sigma_r=sr, boundary=mode, const_val=0.5, cvt=cvt)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float32])
+def test_global_operators_unaligned(gpu, dtype):
+    """Reductions and histograms over rows back to back from any first byte and
+    over pitched rows of every tail length.  Small integers: float sums exact."""
+    f = dtype == np.float32
+    for h, w in ((1, 1), (3, 5), (5, 17), (37, 1003), (64, 255)):
+        src = np.random.default_rng(w).integers(0, 200, (h, w)).astype(dtype)
+        flat = torch.zeros(h * w + 3, dtype=DT[np.dtype(dtype)], device="cuda")
+        for off in (0, 1, 3):
+            flat[off:off + h * w] = to_gpu(src).flatten()
+            for img in (flat[off:off + h * w].view(h, w), _cut(src, off, 2)):
+                for red, ref in ((capi.SUM, src.astype(np.float64).sum()), (capi.MIN, src.min()),
+                                 (capi.MAX, src.max())):
+                    res = torch.zeros(1, dtype=torch.float32 if f else torch.int32, device="cuda")
+                    op.reduce(img, red, res)
+                    assert float(res.item()) == float(ref)
+                bins = torch.zeros(256, dtype=torch.int32, device="cuda")
+                op.histogram(img, 256, bins)
+                np.testing.assert_array_equal(to_host(bins, np.int32),
+                                              np.bincount(src.astype(np.int64).ravel(),
+                                                          minlength=256))
