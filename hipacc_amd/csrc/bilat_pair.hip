@@ -237,6 +237,8 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   const Geom& g = a.g;
   if (g.in_dtype != HIPACC_F32 || g.out_dtype != HIPACC_F32 || g.cvt == HIPACC_CVT_ROUND)
     return HIPACC_ERR_UNSUPPORTED;
+  // scaled pixels stay far from the ends of the float range
+  if (!(a.scale > 1e-15 && a.scale < 1e15)) return HIPACC_ERR_UNSUPPORTED;
   const int kk = a.ksize * a.ksize, r = a.ksize / 2;
   for (int t = 0; t < kk; ++t)
     if (!(a.lsp[t] == a.lsp[kk - 1 - t])) return HIPACC_ERR_UNSUPPORTED;

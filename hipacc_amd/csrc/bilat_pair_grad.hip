@@ -268,6 +268,7 @@ int dispatch_bilat_pair_grad(const BilatGradArgs& a, int* nblocks, hipStream_t s
   }();
   const int r = a.ksize / 2, kk = a.ksize * a.ksize;
   if (!a.gx || !a.sym || r < 2 || r > 4) return HIPACC_ERR_UNSUPPORTED;
+  if (!(a.scale > 1e-15 && a.scale < 1e15)) return HIPACC_ERR_UNSUPPORTED;   // as forward
   const PairGeom pg = pair_geom(a.w, a.h, a.batch, r, cus, kGradBlocks);
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   // Issue slots of a SIMD, both ways, as in dispatch_bilat_pair.
