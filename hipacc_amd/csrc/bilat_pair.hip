@@ -1,17 +1,25 @@
 // bilat_pair.hip -- bilateral filter on float images, each pixel pair's
 // weight evaluated once (hh_bilat_pair.hpp).
 //
-// Per pair of pixels: difference, exponent (one FMA on pixels scaled by
-// sqrt(c log2 e)), exponential (two issue slots) and the four sums of the
-// pair, 8 slots; the tile kernel (bilateral.hip) spends 7 on each of the
-// pair's two taps.  The sums are of d = X(q) - X(p), so that
-// Y(p) = X(p) + SUM s d / SUM s: the rounding of the sums scales with the
-// local contrast instead of the pixel's value (13x13 over 4096^2 pixels in
-// [0, 1]: 3.5e-8 off the 64-bit result in the 2-norm, the tile kernel 2.8e-7).
+// Per pair of pixels: difference, exponent, exponential (two issue slots) and
+// the four sums of the pair; the tile kernel (bilateral.hip) spends 7 slots on
+// each of the pair's two taps.  The sums are of d = X(q) - X(p), so that
+// Y(p) = X(p) + SUM s d / SUM s: their rounding scales with the local contrast
+// instead of the pixel's value (13x13 over 4096^2 pixels in [0, 1]: 3e-8 off
+// the 64-bit result in the 2-norm, the tile kernel 2.8e-7).
 //
-// 4096^2: 13x13 527 -> 405 us, 7x7 175 -> 120 us; 16 x 1024^2 7x7 173 -> 126
-// us (tile kernel -> here); VALU issue bound, 2970 of 3120 slots of a 13x13
-// row in the pairs.
+// RAW forms d from the pixels themselves (halved, so that the difference of
+// any two finite pixels is finite) and the exponent in two instructions, 9
+// slots a pair: the weights and the norm are as exact as the tile kernel's.
+// Without RAW the pixels are scaled by sqrt(c log2 e) first and the exponent
+// is one FMA, 8 slots.  Rounding the scaled pixel moves a weight by its last
+// place times the pixel's size over sigma; the sums of s d hide that below the
+// last place of Y, but the norm, which the backward reads, would show it
+// (pixels 1000 .. 1001 at sigma 0.1: norm 5e-4 off, Y 7e-8).  No value of one
+// pixel enters another's sums in either form except through s.
+//
+// Tile kernel and here, us: 4096^2 13x13 527 and 411, 7x7 175 and 119;
+// 16 x 1024^2 7x7 173 and 125, RAW 137.  VALU issue bound.
 #include <cmath>
 
 #include "hh_bilat_pair.hpp"
@@ -20,7 +28,7 @@ namespace hh {
 
 typedef float pair_f4 __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int R>
+template <int R, bool RAW>
 __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const BilatArgs a, const PairGeom pg) {
   constexpr int V = 4, K = 2 * R + 1, HL = (R + V - 1) / V, NW = V + 2 * R;
   __shared__ __align__(16) float4 part[3][R][2][64];   // first R rows of waves 1..3: den, num
@@ -31,7 +39,6 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
   const float* in = static_cast<const float*>(g.in) + (long long)pl.b * g.in_plane;
   const int yw = pl.y0 + (wave == 0 ? 0 : pg.n0 + (wave - 1) * pg.n);   // first row of the segment
   const int nrow = wave == 0 ? pg.n0 : pg.n;
-  const bool cmode = g.boundary == HIPACC_BOUNDARY_CONSTANT;
   const LaneCols<V> cols = lane_cols<V>(g, g.in_ox + pl.x);
   bool raw = true;   // the lane's 4 pixels are adjacent in memory
 #pragma unroll
@@ -65,15 +72,35 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
     for (int e = 0; e < V; ++e) v[e] = rc || cols.cst[e] ? g.const_f : v[e];
   };
 
-  float ref = 0.0f;                        // pixels are scaled about this value
-  // Factors as sums of two floats: a factor's own rounding would shift sigma
-  // for every pixel alike, where a product rounded once is off at random (the
-  // gradient for sigma is a sum that cancels and shows the difference).
-  const float sc = (float)a.scale, scl = (float)(a.scale - (double)sc);
-  const double inv = 1.0 / a.scale;
+  const float k2 = (float)(-4.0 * a.scale * a.scale);   // RAW: of halved differences
+  const float sc = RAW ? 0.5f : (float)a.scale;
+  // (as the sum of two floats: a factor's own rounding would move every pixel)
+  const double inv = 1.0 / (double)sc;
   const float isc = (float)inv, iscl = (float)(inv - (double)isc);
   const float s0 = __builtin_amdgcn_exp2f(a.lsp[R * K + R]);
-  // x, den, num: scaled pixels of row y and their sums (without the centre tap)
+  // Scaled pixels are held within a limit: a finite pixel must not become
+  // infinite (0 * inf would spread NaN where the weight is 0).  Pixels beyond
+  // it differ by far more than sigma from every other value, so their own
+  // output is the pixel (`limited`, uniform over the wave: some are).
+  constexpr float kLimit = 1e38f;
+  bool limited = false;
+  auto hold = [&](const float (&v)[V], float (&x)[V]) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e] = v[e] * sc;
+    if constexpr (!RAW) {
+      static_assert(V == 4, "pixels per lane");
+      const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])),
+                                      __builtin_fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])));
+      if (__any(m >= kLimit)) {
+        limited = true;
+#pragma unroll
+        for (int e = 0; e < V; ++e)   // (infinities and NaN stay)
+          x[e] = __builtin_fabsf(v[e]) <= 3.402823466e38f
+                     ? __builtin_amdgcn_fmed3f(x[e], -kLimit, kLimit) : v[e];
+      }
+    }
+  };
+  // x, den, num: pixels of row y as held and their sums (without the centre tap)
   auto finish = [&](int y, const float (&x)[V], const float (&den)[V], const float (&num)[V]) {
     if (!pl.store || y >= g.is_h) return;
     float r[V], n[V];
@@ -84,7 +111,7 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
       // bit only scales the correction SUM s d / SUM s
       const float q = s0 > 1e-30f ? num[e] * __builtin_amdgcn_rcpf(n[e]) : num[e] / n[e];
       const float xq = x[e] + q;
-      r[e] = __builtin_fmaf(xq, isc, __builtin_fmaf(xq, iscl, ref));
+      r[e] = RAW ? xq * isc : __builtin_fmaf(xq, isc, xq * iscl);
     }
     float* dst = static_cast<float*>(g.out) + (long long)pl.b * g.out_plane +
                  (long long)(g.out_oy + y) * g.out_stride + g.out_ox + pl.x;
@@ -108,25 +135,16 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
     }
   };
 
-  float xr[R + 1][V], nx[V];               // rows y .. y + R, scaled; row y + R + 1 as loaded
+  float xr[R + 1][V], nx[V];               // rows y .. y + R as held; row y + R + 1 as loaded
   float den[R + 1][V], num[R + 1][V];      // sums of rows y .. y + R
-  auto scaled = [&](const float (&v)[V], float (&x)[V]) {
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const float d = v[e] - ref;
-      x[e] = __builtin_fmaf(d, sc, d * scl);
-    }
-  };
   {
     float v[R + 1][V];
 #pragma unroll
     for (int k = 0; k <= R; ++k) load_row(ys + k, v[k]);
     load_row(ys + R + 1, nx);
-    const float f = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v[0][0])));
-    ref = __builtin_fabsf(f) < 1e30f ? f : 0.0f;
 #pragma unroll
     for (int k = 0; k <= R; ++k) {
-      scaled(v[k], xr[k]);
+      hold(v[k], xr[k]);
 #pragma unroll
       for (int e = 0; e < V; ++e) den[k][e] = num[k][e] = 0.0f;
     }
@@ -163,7 +181,8 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
         for (int e = 0; e < V; ++e) {
           const int m = e + dx + R;
           const float d = win[m] - xr[0][e];
-          const float s = __builtin_amdgcn_exp2f(__builtin_fmaf(-d, d, l));
+          const float s = __builtin_amdgcn_exp2f(RAW ? __builtin_fmaf(d * d, k2, l)
+                                                     : __builtin_fmaf(-d, d, l));
           den[0][e] += s;
           num[0][e] = __builtin_fmaf(s, d, num[0][e]);
           if (dx == first || e == V - 1) {
@@ -207,7 +226,7 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
         den[k][e] = den[k + 1][e];
         num[k][e] = num[k + 1][e];
       }
-    scaled(nx, xr[R]);
+    hold(nx, xr[R]);
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       nx[e] = nn[e];
@@ -224,6 +243,24 @@ __global__ __launch_bounds__(256, R <= 4 ? 4 : 3) void bilat_pair_kernel(const B
       finish(yw + nrow + k, xr[k], d, m);
     }
   }
+  if (!RAW && limited && pl.store) {
+    // outputs this wave wrote of pixels beyond the limit, except NaN ones (an
+    // infinity or a NaN in the window)
+    const int y1 = min(yw + nrow + (wave < 3 ? R : 0), g.is_h);
+    for (int y = yw + (wave == 0 ? 0 : R); y < y1; ++y) {
+      bool rc;
+      const int yy = row_src(g, g.in_oy + y, rc);
+      for (int e = 0; e < V && pl.x + e < g.is_w; ++e) {
+        const LaneCols<1> col = lane_cols<1>(g, g.in_ox + pl.x + e);
+        const float v = rc || col.cst[0] ? g.const_f : in[(long long)yy * g.in_stride + col.x[0]];
+        if (!(__builtin_fabsf(v * sc) >= kLimit)) continue;
+        float* dst = static_cast<float*>(g.out) + (long long)pl.b * g.out_plane +
+                     (long long)(g.out_oy + y) * g.out_stride + g.out_ox + pl.x + e;
+        const float old = *dst;
+        if (old == old) *dst = v;
+      }
+    }
+  }
 }
 
 int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
@@ -237,7 +274,7 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   const Geom& g = a.g;
   if (g.in_dtype != HIPACC_F32 || g.out_dtype != HIPACC_F32 || g.cvt == HIPACC_CVT_ROUND)
     return HIPACC_ERR_UNSUPPORTED;
-  // scaled pixels stay far from the ends of the float range
+  // the exponent's factor stays far from the ends of the float range
   if (!(a.scale > 1e-15 && a.scale < 1e15)) return HIPACC_ERR_UNSUPPORTED;
   const int kk = a.ksize * a.ksize, r = a.ksize / 2;
   for (int t = 0; t < kk; ++t)
@@ -256,9 +293,15 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   const double pair =
       (double)ceil_div(pg.blocks, cus) * (pg.n + 1.0) * (17.8 * kk + 180.0) + 2500.0;
   if (tile < pair) return HIPACC_ERR_UNSUPPORTED;
+  // Scaled pixels only where no norm is asked for, and where scaling neither
+  // takes small pixels below the float range nor large ones to its limit.
+  const bool raw = a.norm || !(a.scale > 1e-3 && a.scale < 1e9);
 #define HH_BP(R)                                                                             \
   case R:                                                                                    \
-    hipLaunchKernelGGL((bilat_pair_kernel<R>), dim3(pg.blocks), dim3(256), 0, s, a, pg);     \
+    if (raw)                                                                                 \
+      hipLaunchKernelGGL((bilat_pair_kernel<R, true>), dim3(pg.blocks), dim3(256), 0, s, a, pg);  \
+    else                                                                                     \
+      hipLaunchKernelGGL((bilat_pair_kernel<R, false>), dim3(pg.blocks), dim3(256), 0, s, a, pg); \
     break;
   switch (r) {
     HH_BP(2) HH_BP(3) HH_BP(4) HH_BP(5) HH_BP(6) HH_BP(7)

@@ -1,0 +1,154 @@
+"""Bilateral filter on images whose pixels differ by orders of magnitude, at
+sizes the pixel-pair kernels take: hot pixels at the first place of the image
+and inside it, a CONSTANT border far from the image, images of one batch in
+different units, values up to the ends of the float range, infinities and NaN.
+Compared with 64 bits, each pixel by a bound relative to what its own window
+may contribute.
+
+Forward bound.  With u = 2^-24 and M = |X(p)| + 8 sigma (a pixel farther from
+X(p) than 8 sigma has a weight below 2^-46 of its place in the window, and its
+product with the difference is smaller still): each of the n = k*k terms
+enters the sums with a few roundings, and a weight s is off by
+s (4 |e| + 2) u for its own exponent e (s |e| <= 0.54) and, where the pixels
+are scaled before the difference is taken, by another s |t| M u / sigma for
+the scaled difference t (s t^2 <= 0.54).  Over the sum of weights, which is at
+least the centre's 1, that is less than 2 (n + 10) u M.  The norm has no
+division by itself: less than 5 (n + 10) u of it."""
+import numpy as np
+import pytest
+import torch
+
+from hipacc_amd import capi, operators as op
+
+pytestmark = pytest.mark.gpu
+
+SIGMA, SIGMA_D = 0.1, 2.0
+U = 2.0 ** -24
+SHAPE = (1, 1501, 2050)
+HOT = [1e2, 1e4, 1e6, 1e9, -9999.0, 3.4028234e38]
+
+
+def _base(shape, seed):
+    return torch.rand(shape, generator=torch.Generator("cuda").manual_seed(seed), device="cuda")
+
+
+def _windows(x, k, mode, cval):
+    """(spatial weight, X(p + o)) of every tap, boundary handling applied, in 64 bits."""
+    r = k // 2
+    h, w = x.shape[-2:]
+
+    def idx(n):
+        i = torch.arange(-r, n + r, device="cuda")
+        out = (i < 0) | (i >= n)
+        if mode == capi.REPEAT:
+            i = i % n
+        elif mode == capi.MIRROR:
+            i = torch.where(i < 0, -i - 1, torch.where(i >= n, 2 * n - 1 - i, i))
+        return i.clamp(0, n - 1), out
+
+    (iy, oy), (ix, ox) = idx(h), idx(w)
+    p = x.double()[..., iy, :][..., ix]
+    if mode == capi.CONSTANT:
+        p = p.masked_fill(oy[:, None] | ox[None, :], float(np.float32(cval)))
+    for dy in range(k):
+        for dx in range(k):
+            sp = np.exp(-((dx - r) ** 2 + (dy - r) ** 2) / (2.0 * SIGMA_D * SIGMA_D))
+            yield float(np.float32(sp)), p[..., dy:dy + h, dx:dx + w]
+
+
+def _exact(x, k, sigma, mode, cval):
+    c = x.double()
+    num, den = torch.zeros_like(c), torch.zeros_like(c)
+    for sp, v in _windows(x, k, mode, cval):
+        s = torch.exp(-(v - c) ** 2 / (2.0 * float(np.float32(sigma)) ** 2)) * sp
+        num += s * v
+        den += s
+    return num / den, den
+
+
+def _run(x, k, sigma, mode, cval, train):
+    y, n = torch.empty_like(x), torch.empty_like(x)
+    if train:
+        op.prepare_bilateral_train(x, y, n, k, SIGMA_D, sigma, boundary=mode,
+                                   const_val=cval).launch()
+    else:
+        op.bilateral(x, y, k, SIGMA_D, sigma, boundary=mode, const_val=cval)
+    torch.cuda.synchronize()
+    return y, n
+
+
+def _check(x, k, sigma, mode, cval, train, where=None):
+    y, n = _run(x, k, sigma, mode, cval, train)
+    ey, en = _exact(x, k, sigma, mode, cval)
+    where = torch.ones_like(x, dtype=torch.bool) if where is None else where
+    t = k * k
+    tol = 2 * (t + 10) * U * (x.double().abs() + 8 * sigma)
+    bad = ~((y.double() - ey).abs() <= tol) & where
+    assert not bad.any(), (int(bad.sum()), ((y.double() - ey).abs() / tol)[where].max().item())
+    if train:
+        bad = ~((n.double() - en).abs() <= 5 * (t + 10) * U * en) & where
+        assert not bad.any(), (int(bad.sum()), ((n.double() - en).abs() / en)[where].max().item())
+
+
+def _mark(x, value):
+    """One marker at the image's first pixel, some inside it, one at its last."""
+    h, w = x.shape[-2:]
+    for y, c in ((0, 0), (0, w - 1), (h // 3, w // 2), (h // 2, 0), (h // 2, w // 2 + 1),
+                 (h - 1, w - 1)):
+        x[..., y, c] = value
+    return x
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("value", HOT)
+@pytest.mark.parametrize("k,mode", [(7, capi.CLAMP), (9, capi.MIRROR), (5, capi.CONSTANT)])
+def test_hot_pixels(gpu, k, mode, value, train):
+    _check(_mark(_base(SHAPE, 1), value), k, SIGMA, mode, 0.5, train)
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("cval", [-9999.0, 1e6, 1e9, 3.4028234e38])
+@pytest.mark.parametrize("k", [5, 7, 13])
+def test_far_constant(gpu, k, cval, train):
+    _check(_base(SHAPE, 2), k, SIGMA, capi.CONSTANT, cval, train)
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_images_of_a_batch_in_different_units(gpu, train):
+    x = _base((5, 517, 1027), 3)
+    x[1] *= 1e6
+    x[3] = -1e9
+    _check(x, 7, SIGMA, capi.CLAMP, 0.0, train)
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("offset,sigma", [(1000.0, 0.1), (1000.0, 0.01), (0.0, 1e-3),
+                                          (0.0, 1e4), (0.0, 1e12)])
+def test_offset_and_sigma(gpu, offset, sigma, train):
+    _check(_base(SHAPE, 4) + offset, 7, sigma, capi.REPEAT, 0.0, train)
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_both_ends_of_the_float_range(gpu, train):
+    """A weight of 0 leaves out even the farthest finite pixel."""
+    x = _mark(_base(SHAPE, 5), 3.4028234e38)
+    x[..., 200:204, 300] = -3.4028234e38
+    x[..., 202, 301] = 3.4028234e38
+    x[..., 800, 900] = 2.0e38
+    _check(x, 7, SIGMA, capi.CLAMP, 0.0, train)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("train", [False, True])
+def test_infinities_and_nan_stay_in_their_windows(gpu, train, value):
+    """A window that holds one gives NaN (0 * inf, as in 64 bits), the others
+    are not touched."""
+    k = 7
+    x = _base(SHAPE, 6)
+    x[..., 0, 0] = value
+    x[..., 700, 1000] = value
+    ey, _ = _exact(x, k, SIGMA, capi.CLAMP, 0.0)
+    y, _ = _run(x, k, SIGMA, capi.CLAMP, 0.0, train)
+    assert torch.equal(torch.isnan(y), torch.isnan(ey))
+    assert torch.isnan(ey).any()
+    _check(x, k, SIGMA, capi.CLAMP, 0.0, train, ~torch.isnan(ey))
