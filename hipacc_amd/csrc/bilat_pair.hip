@@ -277,8 +277,11 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   // the exponent's factor stays far from the ends of the float range
   if (!(a.scale > 1e-15 && a.scale < 1e15)) return HIPACC_ERR_UNSUPPORTED;
   const int kk = a.ksize * a.ksize, r = a.ksize / 2;
+  // The centre's weight must be the table's largest: Y is formed from the
+  // centre pixel, so its last place is part of the error even where the pixel
+  // has little part in Y (no weight at all in a table with a hole there).
   for (int t = 0; t < kk; ++t)
-    if (!(a.lsp[t] == a.lsp[kk - 1 - t])) return HIPACC_ERR_UNSUPPORTED;
+    if (!(a.lsp[t] == a.lsp[kk - 1 - t] && a.lsp[t] <= a.lsp[kk / 2])) return HIPACC_ERR_UNSUPPORTED;
   const PairGeom pg = pair_geom(g.is_w, g.is_h, g.batch, r, cus);
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   // Issue slots of a SIMD, both ways: a tile block is one wave per SIMD of 4

@@ -32,7 +32,13 @@ def _base(shape, seed):
     return torch.rand(shape, generator=torch.Generator("cuda").manual_seed(seed), device="cuda")
 
 
-def _windows(x, k, mode, cval):
+def _table(k):
+    r = np.arange(k) - k // 2
+    d2 = r[:, None] ** 2 + r[None, :] ** 2
+    return np.exp(-d2 / (2.0 * SIGMA_D * SIGMA_D)).astype(np.float32)
+
+
+def _windows(x, k, mode, cval, table=None):
     """(spatial weight, X(p + o)) of every tap, boundary handling applied, in 64 bits."""
     r = k // 2
     h, w = x.shape[-2:]
@@ -50,16 +56,16 @@ def _windows(x, k, mode, cval):
     p = x.double()[..., iy, :][..., ix]
     if mode == capi.CONSTANT:
         p = p.masked_fill(oy[:, None] | ox[None, :], float(np.float32(cval)))
+    table = _table(k) if table is None else table
     for dy in range(k):
         for dx in range(k):
-            sp = np.exp(-((dx - r) ** 2 + (dy - r) ** 2) / (2.0 * SIGMA_D * SIGMA_D))
-            yield float(np.float32(sp)), p[..., dy:dy + h, dx:dx + w]
+            yield float(table[dy, dx]), p[..., dy:dy + h, dx:dx + w]
 
 
-def _exact(x, k, sigma, mode, cval):
+def _exact(x, k, sigma, mode, cval, table=None):
     c = x.double()
     num, den = torch.zeros_like(c), torch.zeros_like(c)
-    for sp, v in _windows(x, k, mode, cval):
+    for sp, v in _windows(x, k, mode, cval, table):
         s = torch.exp(-(v - c) ** 2 / (2.0 * float(np.float32(sigma)) ** 2)) * sp
         num += s * v
         den += s
@@ -152,3 +158,23 @@ def test_infinities_and_nan_stay_in_their_windows(gpu, train, value):
     assert torch.equal(torch.isnan(y), torch.isnan(ey))
     assert torch.isnan(ey).any()
     _check(x, k, SIGMA, capi.CLAMP, 0.0, train, ~torch.isnan(ey))
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("centre", [0.0, 1e-4])
+def test_tables_with_a_small_centre(gpu, train, centre):
+    """A pixel far from its neighbours that has little part in its own output:
+    the image is not negative, so the sums' error is relative to Y."""
+    k, sigma = 7, 1e7
+    table = _table(k)
+    table[k // 2, k // 2] = centre
+    x = _mark(_base(SHAPE, 7), 1e6)
+    y, n = torch.empty_like(x), torch.empty_like(x)
+    if train:
+        op.prepare_bilateral_train(x, y, n, k, SIGMA_D, sigma, spatial=table,
+                                   boundary=capi.CLAMP).launch()
+    else:
+        op.bilateral(x, y, k, SIGMA_D, sigma, spatial=table, boundary=capi.CLAMP)
+    ey, _ = _exact(x, k, sigma, capi.CLAMP, 0.0, table)
+    err = (y.double() - ey).abs() / ey
+    assert (err <= 2 * (k * k + 10) * U).all(), err.max().item()
