@@ -2,18 +2,23 @@
 // with each pixel pair evaluated once, in the lane layout of
 // hh_bilat_pair.hpp.
 //
-// With D = X(q) - X(p) scaled by sqrt(c log2 e), a = dY / norm and
-// z = X - Y, the pair's weight s serves four sums: the centre terms of both
-// pixels (S2 = SUM s D^2 and, for dL/dc, S3 = SUM s D^3 towards the
-// neighbour) and the neighbour term of each (through the other's a and a z):
-//   N(q) += a(p) s [1 - k D^2] - b(p) s D      b = k sqrt(c log2 e) a z, k = 2 ln 2
-//   N(p) += a(q) s [1 - k D^2] + b(q) s D
-//   dX(t) = N(t) + a(t) s(centre) + k a(t) S2(t) - 2c z(t)^2 dY(t)
-//   dL/dc = -(c log2 e)^(-3/2) SUM_t [a(t) S3(t) + b(t) S2(t) / k]
+// With D = X(q) - X(p), a = dY / norm, z = X - Y and b = 2c a z, the pair's
+// weight s serves four sums: the centre terms of both pixels (S2 = SUM s D^2
+// and, for dL/dc, S3 = SUM s D^3 towards the neighbour) and the neighbour term
+// of each (through the other's a and b):
+//   N(q) += a(p) s [1 - 2c D^2] - b(p) s D
+//   N(p) += a(q) s [1 - 2c D^2] + b(q) s D
+//   dX(t) = N(t) + a(t) s(centre) + 2c a(t) S2(t) - 2c z(t)^2 dY(t)
+//   dL/dc = -SUM_t [a(t) S3(t) + a(t) z(t) S2(t)]
 // The last term of dX is the centre term's product with SUM s (X(q) - X(t)),
-// which the forward gave as (Y - X) norm.  17 issue slots a pair against 13 a
-// tap in the tile kernel: 7x7 at 16 x 1024^2 367 -> 274 us (CONSTANT,
-// without a halo ring), VALU issue bound.
+// which the forward gave as (Y - X) norm.  Differences are those of the pixels
+// themselves (halved, so that the difference of any two finite pixels is
+// finite), and every product starts with s: a weight of 0 leaves out a
+// neighbour however far its value is.
+//
+// 17 issue slots a pair against 13 a tap in the tile kernel: 7x7 at
+// 16 x 1024^2 367 us there, 267 here (CONSTANT, without a halo ring), VALU
+// issue bound.
 #include <cmath>
 
 #include "hh_bilat_pair.hpp"
@@ -25,9 +30,8 @@ typedef float pair_f4 __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int R>
 __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGradArgs a,
-                                                                              const PairGeom pg) {
+                                                                 const PairGeom pg) {
   constexpr int V = 4, K = 2 * R + 1, HL = (R + V - 1) / V, NW = V + 2 * R;
-  constexpr float kKappa = 1.38629436111989061883f;   // 2 ln 2
   __shared__ __align__(16) float4 part[3][R][3][64];  // first R rows of waves 1..3: N, S2, S3
   __shared__ double red[4];
   const int lane = threadIdx.x & 63;
@@ -88,10 +92,9 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
     }
   };
 
-  const float sc = (float)a.scale, scl = (float)(a.scale - (double)sc);   // as in bilat_pair_kernel
-  const float s0 = a.sp[R * K + R], c2 = 2.0f * a.c, bsc = kKappa * sc;
-  const double zsc = a.scale / (double)bsc;   // b * zsc = a z sqrt(c log2 e)
-  float ref = 0.0f;
+  // of halved differences h: s = 2^(l + k2 h^2), 2c D^2 = c8 h^2, b D = (4c a z) h
+  const float k2 = (float)(-4.0 * a.scale * a.scale), c8 = 8.0f * a.c, c4 = 4.0f * a.c, c2 = 2.0f * a.c;
+  const float s0 = a.sp[R * K + R];
   float xr[R + 1][V], ar[R + 1][V], br[R + 1][V];      // rows y .. y + R
   float nn[R + 1][V], s2[R + 1][V], s3[R + 1][V];      // their sums
   // a loaded row becomes row k of the window; N starts with the terms of the
@@ -101,15 +104,15 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       const float av = r.g[e] / r.d[e], z = r.x[e] - r.y[e];
-      const float xd = r.x[e] - ref;
-      xr[k][e] = __builtin_fmaf(xd, sc, xd * scl);
+      xr[k][e] = 0.5f * r.x[e];
       ar[k][e] = av;
-      br[k][e] = av * (z * bsc);
+      br[k][e] = c4 * (av * z);
       nn[k][e] = own ? __builtin_fmaf(-c2 * z * z, r.g[e], av * s0) : 0.0f;
       s2[k][e] = 0.0f;
       s3[k][e] = 0.0f;
     }
   };
+  const double rc = 1.0 / (double)a.c;
   double dc = 0.0;   // the two terms cancel largely, and the pixels' sums too
   auto finish = [&](int y, const float (&av)[V], const float (&bv)[V], const float (&n)[V],
                     const float (&t2)[V], const float (&t3)[V]) {
@@ -117,9 +120,10 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
     float v[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-      v[e] = __builtin_fmaf(kKappa * av[e], t2[e], n[e]);
-      // a and b are 0 for the columns beside the image
-      dc += (double)av[e] * (double)t3[e] + zsc * ((double)bv[e] * (double)t2[e]);
+      v[e] = __builtin_fmaf(c8 * av[e], t2[e], n[e]);
+      // a and b are 0 for the columns beside the image; D^3 = 8 h^3, and
+      // a z D^2 = b h^2 / c in the halved differences' b
+      dc += 8.0 * ((double)av[e] * (double)t3[e]) + rc * ((double)bv[e] * (double)t2[e]);
     }
     float* dst = a.gx + (long long)pl.b * a.gx_plane + (long long)y * a.gx_stride + pl.x;
     if (pl.x + V <= a.w) {
@@ -138,9 +142,6 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
 #pragma unroll
     for (int k = 0; k <= R; ++k) load_row(ys + k, r[k]);
     load_row(ys + R + 1, nx);
-    const float f = __builtin_bit_cast(
-        float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, r[0].x[0])));
-    ref = __builtin_fabsf(f) < 1e30f ? f : 0.0f;
 #pragma unroll
     for (int k = 0; k <= R; ++k) enter(r[k], k, wave == 0 || k == R);
   }
@@ -176,9 +177,9 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
         for (int e = 0; e < V; ++e) {
           const int m = e + dx + R;
           const float d = wx[m] - xr[0][e];
-          const float dd = d * d;
-          const float s = __builtin_amdgcn_exp2f(l - dd);
-          const float sp = s * __builtin_fmaf(-kKappa, dd, 1.0f), sd = s * d, t2 = s * dd;
+          const float s = __builtin_amdgcn_exp2f(__builtin_fmaf(d * d, k2, l));
+          const float sd = s * d, t2 = sd * d;
+          const float sp = __builtin_fmaf(-c8, t2, s);
           nn[0][e] = __builtin_fmaf(wa[m], sp, nn[0][e]);
           nn[0][e] = __builtin_fmaf(wb[m], sd, nn[0][e]);
           s2[0][e] += t2;
@@ -251,11 +252,8 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
   for (int off = 32; off >= 1; off >>= 1) dc += __shfl_xor(dc, off, 64);
   if (lane == 0) red[wave] = dc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const double isc = 1.0 / a.scale;
-    a.partials[blockIdx.x] =
-        (float)(-(((red[0] + red[1]) + red[2]) + red[3]) * (isc * isc * isc));
-  }
+  if (threadIdx.x == 0)
+    a.partials[blockIdx.x] = (float)(-(((red[0] + red[1]) + red[2]) + red[3]));
 }
 
 int dispatch_bilat_pair_grad(const BilatGradArgs& a, int* nblocks, hipStream_t s) {

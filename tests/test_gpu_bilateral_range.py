@@ -13,11 +13,16 @@ s (4 |e| + 2) u for its own exponent e (s |e| <= 0.54) and, where the pixels
 are scaled before the difference is taken, by another s |t| M u / sigma for
 the scaled difference t (s t^2 <= 0.54).  Over the sum of weights, which is at
 least the centre's 1, that is less than 2 (n + 10) u M.  The norm has no
-division by itself: less than 5 (n + 10) u of it."""
+division by itself: less than 5 (n + 10) u of it.
+
+The backward is held to the adjoint tests' bound, 1e-5 of the sum of
+magnitudes, which is itself a sum over the pixel's window."""
 import numpy as np
 import pytest
 import torch
 
+import oracle_binding as ob
+from gpu_util import to_host
 from hipacc_amd import capi, operators as op
 
 pytestmark = pytest.mark.gpu
@@ -178,3 +183,45 @@ def test_tables_with_a_small_centre(gpu, train, centre):
     ey, _ = _exact(x, k, sigma, capi.CLAMP, 0.0, table)
     err = (y.double() - ey).abs() / ey
     assert (err <= 2 * (k * k + 10) * U).all(), err.max().item()
+
+
+GRAD_SHAPE = (3, 620, 1030)
+
+
+def _check_grad(x, g, k, mode, cval, images=None):
+    y, n, gx = torch.empty_like(x), torch.empty_like(x), torch.full_like(x, 7.0)
+    gs = torch.zeros(1, device="cuda")
+    op.prepare_bilateral_train(x, y, n, k, SIGMA_D, SIGMA, boundary=mode, const_val=cval).launch()
+    op.prepare_bilateral_grad(x, y, n, g, gx, k, SIGMA_D, SIGMA, grad_sigma=gs, boundary=mode,
+                              const_val=cval).launch()
+    dx, ds, dxa, dsa = ob.bilateral_grad(to_host(x, np.float32), to_host(g, np.float32), k,
+                                         SIGMA_D, SIGMA, boundary=mode, const_val=cval,
+                                         with_abs=True)
+    err = np.abs(to_host(gx, np.float32) - dx)
+    for b in range(x.shape[0]) if images is None else images:
+        assert (err[b] <= 1e-5 * dxa[b] + 1e-12).all(), (b, (err[b] / (dxa[b] + 1e-30)).max())
+    assert abs(float(gs.item()) - ds) <= 1e-5 * dsa
+
+
+def _gy(shape, seed):
+    return torch.randn(shape, generator=torch.Generator("cuda").manual_seed(seed), device="cuda")
+
+
+@pytest.mark.parametrize("value", HOT)
+@pytest.mark.parametrize("k,mode", [(7, capi.CLAMP), (9, capi.MIRROR), (5, capi.CONSTANT)])
+def test_hot_pixels_backward(gpu, k, mode, value):
+    _check_grad(_mark(_base(GRAD_SHAPE, 11), value), _gy(GRAD_SHAPE, 12), k, mode, 0.5)
+
+
+@pytest.mark.parametrize("cval", [-9999.0, 1e6, 1e9, 3.4028234e38])
+def test_far_constant_backward(gpu, cval):
+    _check_grad(_base(GRAD_SHAPE, 13), _gy(GRAD_SHAPE, 14), 7, capi.CONSTANT, cval)
+
+
+def test_images_of_a_batch_in_different_units_backward(gpu):
+    """The image in other units takes no gradient: its own dX and part of
+    dL/dsigma are 0, the other images' are theirs."""
+    x, g = _base(GRAD_SHAPE, 15), _gy(GRAD_SHAPE, 16)
+    x[1] *= 1e6
+    g[1] = 0.0
+    _check_grad(x, g, 7, capi.REPEAT, 0.0)
