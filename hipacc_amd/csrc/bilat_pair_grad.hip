@@ -3,21 +3,22 @@
 // hh_bilat_pair.hpp.
 //
 // With D = X(q) - X(p), a = dY / norm, z = X - Y and b = 2c a z, the pair's
-// weight s serves four sums: the centre terms of both pixels (S2 = SUM s D^2
-// and, for dL/dc, S3 = SUM s D^3 towards the neighbour) and the neighbour term
-// of each (through the other's a and b):
-//   N(q) += a(p) s [1 - 2c D^2] - b(p) s D
-//   N(p) += a(q) s [1 - 2c D^2] + b(q) s D
-//   dX(t) = N(t) + a(t) s(centre) + 2c a(t) S2(t) - 2c z(t)^2 dY(t)
+// weight s serves the centre terms of both pixels (S2 = SUM s D^2 and, for
+// dL/dc, S3 = SUM s D^3 towards the neighbour, and the pixel's own b with
+// SUM s D) and the neighbour term of each (through the other's a and b):
+//   N(q) += a(p) s [1 - 2c D^2] - [b(p) + b(q)] s D
+//   N(p) += a(q) s [1 - 2c D^2] + [b(q) + b(p)] s D
+//   dX(t) = N(t) + a(t) s(centre) + 2c a(t) S2(t)
 //   dL/dc = -SUM_t [a(t) S3(t) + a(t) z(t) S2(t)]
-// The last term of dX is the centre term's product with SUM s (X(q) - X(t)),
-// which the forward gave as (Y - X) norm.  Differences are those of the pixels
-// themselves (halved, so that the difference of any two finite pixels is
-// finite), and every product starts with s: a weight of 0 leaves out a
-// neighbour however far its value is.
+// (SUM s D is also (Y - X) norm, which would save the addition of the two b,
+// but -2c z^2 dY in its place squares the rounding of Y: an image of 1e6, flat
+// over the window, with Y one last place off would get 0.4 dY for 0.)
+// Differences are those of the pixels themselves (halved, so that the
+// difference of any two finite pixels is finite), and every product starts
+// with s: a weight of 0 leaves out a neighbour however far its value is.
 //
-// 17 issue slots a pair against 13 a tap in the tile kernel: 7x7 at
-// 16 x 1024^2 367 us there, 267 here (CONSTANT, without a halo ring), VALU
+// 18 issue slots a pair against 13 a tap in the tile kernel: 7x7 at
+// 16 x 1024^2 367 us there, 276 here (CONSTANT, without a halo ring), VALU
 // issue bound.
 #include <cmath>
 
@@ -93,21 +94,21 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
   };
 
   // of halved differences h: s = 2^(l + k2 h^2), 2c D^2 = c8 h^2, b D = (4c a z) h
-  const float k2 = (float)(-4.0 * a.scale * a.scale), c8 = 8.0f * a.c, c4 = 4.0f * a.c, c2 = 2.0f * a.c;
+  const float k2 = (float)(-4.0 * a.scale * a.scale), c8 = 8.0f * a.c, c4 = 4.0f * a.c;
   const float s0 = a.sp[R * K + R];
   float xr[R + 1][V], ar[R + 1][V], br[R + 1][V];      // rows y .. y + R
   float nn[R + 1][V], s2[R + 1][V], s3[R + 1][V];      // their sums
-  // a loaded row becomes row k of the window; N starts with the terms of the
-  // pixel alone (own; the first R rows of waves 1..3 start with them in the
+  // a loaded row becomes row k of the window; N starts with the term of the
+  // pixel alone (own; the first R rows of waves 1..3 start with it in the
   // wave above)
   auto enter = [&](const Row& r, int k, bool own) {
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-      const float av = r.g[e] / r.d[e], z = r.x[e] - r.y[e];
+      const float av = r.g[e] / r.d[e];
       xr[k][e] = 0.5f * r.x[e];
       ar[k][e] = av;
-      br[k][e] = c4 * (av * z);
-      nn[k][e] = own ? __builtin_fmaf(-c2 * z * z, r.g[e], av * s0) : 0.0f;
+      br[k][e] = c4 * (av * (r.x[e] - r.y[e]));
+      nn[k][e] = own ? av * s0 : 0.0f;
       s2[k][e] = 0.0f;
       s3[k][e] = 0.0f;
     }
@@ -179,9 +180,9 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
           const float d = wx[m] - xr[0][e];
           const float s = __builtin_amdgcn_exp2f(__builtin_fmaf(d * d, k2, l));
           const float sd = s * d, t2 = sd * d;
-          const float sp = __builtin_fmaf(-c8, t2, s);
+          const float sp = __builtin_fmaf(-c8, t2, s), bs = wb[m] + br[0][e];
           nn[0][e] = __builtin_fmaf(wa[m], sp, nn[0][e]);
-          nn[0][e] = __builtin_fmaf(wb[m], sd, nn[0][e]);
+          nn[0][e] = __builtin_fmaf(bs, sd, nn[0][e]);
           s2[0][e] += t2;
           s3[0][e] = __builtin_fmaf(t2, d, s3[0][e]);
           if (dx == first || e == V - 1) {
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(256, 2) void bilat_pair_grad_kernel(const BilatGrad
             o2[m] += t2;
             o3[m] = __builtin_fmaf(-t2, d, o3[m]);
           }
-          on[m] = __builtin_fmaf(-br[0][e], sd, on[m]);
+          on[m] = __builtin_fmaf(-bs, sd, on[m]);
         }
         // one offset later: a DPP read right after the write would wait
 #pragma unroll

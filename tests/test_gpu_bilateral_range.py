@@ -225,3 +225,22 @@ def test_images_of_a_batch_in_different_units_backward(gpu):
     x[1] *= 1e6
     g[1] = 0.0
     _check_grad(x, g, 7, capi.REPEAT, 0.0)
+
+
+def test_backward_takes_outputs_rounded_by_any_kernel(gpu):
+    """A flat image of large values with Y one last place off (a quotient of
+    sums may be): every difference is 0, so dX is the weights' own adjoint and
+    dL/dsigma is 0."""
+    k = 7
+    x, g = torch.full(GRAD_SHAPE, 1e6, device="cuda"), _gy(GRAD_SHAPE, 18)
+    y, n, gx = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
+    gs = torch.zeros(1, device="cuda")
+    op.prepare_bilateral_train(x, y, n, k, SIGMA_D, SIGMA, boundary=capi.CLAMP).launch()
+    y = torch.nextafter(x, 2 * x)
+    op.prepare_bilateral_grad(x, y, n, g, gx, k, SIGMA_D, SIGMA, grad_sigma=gs,
+                              boundary=capi.CLAMP).launch()
+    dx, _, dxa, _ = ob.bilateral_grad(to_host(x, np.float32), to_host(g, np.float32), k, SIGMA_D,
+                                      SIGMA, boundary=capi.CLAMP, with_abs=True)
+    err = np.abs(to_host(gx, np.float32) - dx)
+    assert (err <= 1e-5 * dxa + 1e-12).all(), (err / dxa).max()
+    assert float(gs.item()) == 0.0
