@@ -282,20 +282,24 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   // has little part in Y (no weight at all in a table with a hole there).
   for (int t = 0; t < kk; ++t)
     if (!(a.lsp[t] == a.lsp[kk - 1 - t] && a.lsp[t] <= a.lsp[kk / 2])) return HIPACC_ERR_UNSUPPORTED;
-  const PairGeom pg = pair_geom(g.is_w, g.is_h, g.batch, r, cus);
-  if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   // Issue slots of a SIMD, both ways: a tile block is one wave per SIMD of 4
   // pixels x 7 slots a tap, a row of this kernel 4 pixels x 8.9 slots a pair
-  // (both plus staging), and its first rows' loads are waited for.  The long
+  // (both plus staging).  One block per CU waits for each row's loads and for
+  // the pairs' chains, which more blocks hide: 250 slots a row.  The long
   // segments lose where the image does not fill the device a few times over
-  // (us, tile and pair): 7x7 at 1001x751 13.1 and 14.2, at 1920x1080 24.0 and
-  // 24.4, at 2048^2 46 and 36.5; 13x13 at 1024^2 38 and 41, at 1920x1080 69
-  // and 64, at 2048^2 136 and 113.
+  // (us, tile and pair): 5x5 at 1920x1080 16.0 and 18.0, at 4 x 1024^2 29.6
+  // and 31.7, at 1500^2 17.4 and 16.2; 7x7 at 1001x751 12.9 and 14.7, at
+  // 1920x1080 24.7 and 25.5, at 1500^2 28.8 and 23.6; 13x13 at 1024^2 38 and
+  // 43, at 1920x1080 69 and 66, at 2048^2 137 and 116.  RAW costs the pair
+  // kernel up to a tenth of that and moves no line between the two sizes.
   const double tile = (double)ceil_div(ceil_div(g.is_w, 64) * ceil_div(g.is_h, 16) * g.batch, cus) *
                       (28.0 * kk + 300.0);
-  const double pair =
-      (double)ceil_div(pg.blocks, cus) * (pg.n + 1.0) * (17.8 * kk + 180.0) + 2500.0;
-  if (tile < pair) return HIPACC_ERR_UNSUPPORTED;
+  const double row = 17.8 * kk + 180.0, first = 500.0, alone = 250.0;
+  const PairGeom pg = pair_geom(g.is_w, g.is_h, g.batch, r, cus);
+  if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
+  const int rounds = ceil_div(pg.blocks, cus);
+  if (tile < rounds * (pg.n + 1.0) * (row + (rounds == 1 ? alone : 0.0)) + first)
+    return HIPACC_ERR_UNSUPPORTED;
   // Scaled pixels only where no norm is asked for, and where scaling neither
   // takes small pixels below the float range nor large ones to its limit.
   const bool raw = a.norm || !(a.scale > 1e-3 && a.scale < 1e9);
