@@ -282,6 +282,7 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   // has little part in Y (no weight at all in a table with a hole there).
   for (int t = 0; t < kk; ++t)
     if (!(a.lsp[t] == a.lsp[kk - 1 - t] && a.lsp[t] <= a.lsp[kk / 2])) return HIPACC_ERR_UNSUPPORTED;
+  if (r < 2 || r > 7) return HIPACC_ERR_UNSUPPORTED;
   // Issue slots of a SIMD, both ways: a tile block is one wave per SIMD of 4
   // pixels x 7 slots a tap, a row of this kernel 4 pixels x 8.9 slots a pair
   // (both plus staging).  One block per CU waits for each row's loads and for
@@ -295,6 +296,8 @@ int dispatch_bilat_pair(const BilatArgs& a, hipStream_t s) {
   const double tile = (double)ceil_div(ceil_div(g.is_w, 64) * ceil_div(g.is_h, 16) * g.batch, cus) *
                       (28.0 * kk + 300.0);
   const double row = 17.8 * kk + 180.0, first = 500.0, alone = 250.0;
+  // (the shortest segments, before the search for the best ones)
+  if (tile < (kPairRows + 1.0) * row + first) return HIPACC_ERR_UNSUPPORTED;
   const PairGeom pg = pair_geom(g.is_w, g.is_h, g.batch, r, cus);
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   const int rounds = ceil_div(pg.blocks, cus);

@@ -274,6 +274,7 @@ int dispatch_bilat_pair_grad(const BilatGradArgs& a, int* nblocks, hipStream_t s
   // at 2048^2 98 and 82; 9x9 at 1024^2 40.6 and 43.0, at 1500^2 79.5 and 74.4.
   const double tile = (double)ceil_div(a.ntiles, cus) * (52.0 * kk + 900.0);
   const double row = 34.0 * kk + 300.0, first = 4000.0;
+  if (tile < (kPairRows + 1.0) * row + first) return HIPACC_ERR_UNSUPPORTED;
   const PairGeom pg = pair_geom(a.w, a.h, a.batch, r, cus, kGradBlocks);
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
   if (tile < ceil_div(pg.blocks, cus) * (pg.n + 1.0) * row + first) return HIPACC_ERR_UNSUPPORTED;

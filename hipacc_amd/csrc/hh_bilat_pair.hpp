@@ -39,6 +39,8 @@ struct PairGeom {
   int blocks;
 };
 
+constexpr int kPairRows = 4;   // of a segment, at least
+
 // Rows of a wave: the first wave's segment is shorter by the time of the rows
 // it walks above it (half of their pairs).  n minimises the blocks a CU gets x
 // the rows of a wave, with 1.5 rows for a segment's start and end.
@@ -46,7 +48,7 @@ static inline PairGeom pair_geom(int w, int h, int batch, int r, int cus, int mo
   PairGeom best{};
   const int hl = (r + 3) / 4, s = 64 - 2 * hl;
   double bt = 0.0;
-  for (int n = r > 4 ? r : 4; n <= 512; n += n < 128 ? 1 : 16) {
+  for (int n = r > kPairRows ? r : kPairRows; n <= 512; n += n < 128 ? 1 : 16) {
     PairGeom p;
     p.groups = ceil_div(w, 4);
     p.lb = p.groups + 2 * hl;
