@@ -64,15 +64,13 @@ def view(t: torch.Tensor, window: Window = None, dtype: Optional[int] = None) ->
     return v
 
 
-# The raw handle of torch's current stream on the current device, without the
-# Stream object of torch.cuda.current_stream() (2 us of a small operator's
-# 6 us call).
-_device = torch._C._cuda_getDevice
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
 def _stream() -> int:
-    return _raw_stream(_device())
+    # The raw handle of torch's current stream on the current device, without
+    # the Stream object of torch.cuda.current_stream() (2 us of a small
+    # operator's 6 us call).  Looked up at the launch: a torch built without a
+    # GPU has neither name, and the entries that need no device run there too.
+    c = torch._C
+    return c._cuda_getCurrentRawStream(c._cuda_getDevice())
 
 
 class Call:

@@ -5,6 +5,7 @@ import ctypes
 import json
 import re
 import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -140,3 +141,14 @@ def test_adjoint_ring_and_band_enumerations(tmp_path):
     assert p.returncode == 0, p.stderr[-3000:]
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
+
+
+def test_operators_import_on_a_torch_without_a_gpu():
+    """Entries that need no device work on a torch that has no CUDA bindings."""
+    code = ("import torch\n"
+            "for n in ('_cuda_getDevice', '_cuda_getCurrentRawStream'):\n"
+            "    delattr(torch._C, n)\n"
+            "from hipacc_amd import operators as op\n"
+            "print(op.pyramid_plan_tiles([(64, 64)], 3))\n")
+    p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert p.returncode == 0, p.stderr[-2000:]
