@@ -74,7 +74,7 @@ def test_plan_tiles_fit_on_benchmark_geometry(tile_rows):
         # every pixel of level l is covered exactly once by the two lists
         if wide[l]:
             assert wide[l] == sum(-(-(h >> l) // 32) * -(-(w >> l) // 128) for h, w in shapes
-                                  if (h >> l) >= 9 and (w >> l) >= 9)
+                                  if (h >> l) >= 32 and (w >> l) >= 32)
         else:
             assert narrow[l] == sum(-(-(h >> l) // tile_rows) * -(-(w >> l) // 64)
                                     for h, w in shapes)
@@ -88,6 +88,20 @@ def test_plan_tiles_mixed_threshold_geometry():
     narrow, wide = op.pyramid_plan_tiles(tw.MIXED, tw.MIXED_LEVELS)
     assert wide[0] >= 512 and wide[1] >= 512, wide
     assert narrow[1] > 0, narrow   # the 8-row image of level 1 takes narrow tiles
+
+
+def test_plan_tiles_smallest_wide_images():
+    """Images of 31, 32 and 33 pixels a side next to a wide level's large ones:
+    32 x 32 is the smallest that takes wide tiles, and every tile fits."""
+    from hipacc_amd import operators as op
+    import test_gpu_pyramid_wide as tw
+    narrow, wide = op.pyramid_plan_tiles(tw.EDGE, tw.MIXED_LEVELS)
+    assert wide[1] == sum(tw.EDGE_WIDE), wide
+    at1 = [(h >> 1, w >> 1) for h, w in tw.EDGE]
+    assert [n > 0 for n in tw.EDGE_WIDE] == [h >= 32 and w >= 32 for h, w in at1]
+    for a in (31, 32, 33, 34, 35, 63, 65):
+        for b in (31, 32, 33, 129, 257):
+            op.pyramid_plan_tiles([(4096, 4096), (a, b), (b, a)], 3)   # raises if one does not
 
 
 def test_plan_tiles_rejects_bad_sizes():

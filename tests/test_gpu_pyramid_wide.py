@@ -1,8 +1,10 @@
 """The batched pyramid on the geometry where the plan runs levels on wide
 (128 x 32) tiles: at least 512 of them at a level.  Bit-exact against the
 oracle's per-level kernel sequence, with and without contraction, CLAMP and
-MIRROR: 8 levels over large and odd-sized images, and a 4-level set where
-images of 8 and 9 rows share a wide level with 2048^2 images."""
+MIRROR: 8 levels over large and odd-sized images, and 4-level sets where
+small images share a wide level with 2048^2 images: of 8 and 9 rows (narrow
+tiles), and of 31, 32 and 33 on either side of the wide tiles' smallest image,
+32 x 32, whose NN step (33 / 16) is the largest a wide tile is sized for."""
 import numpy as np
 import pytest
 import torch
@@ -16,6 +18,10 @@ LARGE = [(2048, 2048), (2161, 4097), (1151, 1160), (1999, 1001)]
 LARGE_LEVELS = 8
 MIXED = [(2048, 2048), (2048, 2048), (17, 600), (19, 37), (18, 18), (33, 9)]
 MIXED_LEVELS = 4
+# at level 1: 31x300, 32x35, 33x33, 32x500, 31x32, 500x33, 33x31
+EDGE = [(2048, 2048), (2048, 2048), (62, 600), (64, 70), (67, 66), (65, 1001), (63, 64),
+        (1000, 67), (66, 62)]
+EDGE_WIDE = [2048 * 2048 // 4 // (128 * 32)] * 2 + [0, 1, 2, 4, 0, 16, 0]   # tiles at level 1
 
 
 def _run(shapes, levels, mode, fma, seed):
@@ -59,3 +65,13 @@ def test_wide_tiles_mixed_threshold(gpu, mode, fma):
     assert wide[1] >= 512 and narrow[1] > 0, (narrow, wide)
     print(f"wide-tile pyramid mixed mode={mode} fma={fma} wide={wide} narrow={narrow}", flush=True)
     _run(MIXED, MIXED_LEVELS, mode, fma, 950)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [capi.CLAMP, capi.MIRROR])
+@pytest.mark.parametrize("fma", [True, False])
+def test_wide_tiles_smallest_images(gpu, mode, fma):
+    narrow, wide = op.pyramid_plan_tiles(EDGE, MIXED_LEVELS)
+    assert wide[1] == sum(EDGE_WIDE) and narrow[1] > 0, (narrow, wide)
+    print(f"wide-tile pyramid edge mode={mode} fma={fma} wide={wide} narrow={narrow}", flush=True)
+    _run(EDGE, MIXED_LEVELS, mode, fma, 970)
