@@ -420,7 +420,6 @@ static int prep_local(const hipacc_local_desc* d, LocalArgs& a, int& accf, bool&
   a.wdev = d->use_weights ? d->weights_dev : nullptr;
   const int ebi = dtype_bytes(d->in.dtype), ebo = dtype_bytes(d->out.dtype);
   const int vec = 16 / ebi;
-  a.in_vec_ok = rows_aligned(d->in, 16) && (d->in.offset_x % vec) == 0;
   a.out_vec_ok = rows_aligned(d->out, std::min(16, vec * ebo));
   // An integer SUM over a full all-ones window (a box sum) is the outer
   // product of two all-ones rows; integer sums are exact in any order, so
@@ -438,7 +437,6 @@ static int prep_local(const hipacc_local_desc* d, LocalArgs& a, int& accf, bool&
     for (int i = 0; i < sa.kx; ++i) sa.rowi[i] = 1;
     for (int i = 0; i < sa.ky; ++i) sa.coli[i] = 1;
     sa.box = 1;
-    sa.in_vec_ok = a.in_vec_ok;
     sa.out_vec_ok = a.out_vec_ok;
   }
   return HIPACC_OK;
@@ -480,7 +478,6 @@ static int prep_separable(const hipacc_separable_desc* d, SepArgs& a, int& accf)
   }
   const int ebi = dtype_bytes(d->in.dtype), ebo = dtype_bytes(d->out.dtype);
   const int vec = 16 / ebi;
-  a.in_vec_ok = rows_aligned(d->in, 16) && (d->in.offset_x % vec) == 0;
   a.out_vec_ok = rows_aligned(d->out, std::min(16, vec * ebo));
   return HIPACC_OK;
 }
@@ -1058,7 +1055,6 @@ int hipacc_hip_bilateral(const hipacc_bilateral_desc* d, void* stream) {
   const float c_r = 0.5f / (d->sigma_r * d->sigma_r);
   a.k2 = -c_r * 1.44269504088896340736f;
   a.scale = bilat_scale(d->sigma_r);
-  a.in_vec_ok = d->in.dtype == HIPACC_F32 && rows_aligned(d->in, 16) && (d->in.offset_x % 4) == 0;
   a.out_vec_ok = rows_aligned(d->out, 4 * dtype_bytes(d->out.dtype));
   hipStream_t s = static_cast<hipStream_t>(stream);
   Timer tm(s);
@@ -1306,7 +1302,6 @@ int hipacc_hip_bilateral_train(const hipacc_bilateral_grad_desc* d, void* stream
   const float c_r = 0.5f / (d->sigma_r * d->sigma_r);
   a.k2 = -c_r * 1.44269504088896340736f;
   a.scale = bilat_scale(d->sigma_r);
-  a.in_vec_ok = rows_aligned(d->in, 16);
   a.out_vec_ok = rows_aligned(d->out, 16);
   a.norm = static_cast<float*>(d->norm.data);
   a.norm_plane = d->norm.plane_stride;

@@ -39,7 +39,7 @@ struct LocalArgs {
   int reduce;
   int use_weights;
   int fma;          // fp_contract
-  int in_vec_ok;    // input window admits aligned 16-byte row loads (direct loads to LDS)
+  int in_vec_ok;    // input window admits aligned row loads (set by the launches that use it)
   int out_vec_ok;   // output window admits aligned vector stores
   const float* wdev;
   uint8_t domain[kMaxTaps];
@@ -95,7 +95,7 @@ int dispatch_sum_int(const LocalArgs& a, int ppt, hipStream_t s);
 struct SepArgs {
   Geom g;
   int kx, ky;
-  int in_vec_ok, out_vec_ok;
+  int out_vec_ok;
   float rowf[2 * HIPACC_MAX_SEP_RADIUS + 1];
   float colf[2 * HIPACC_MAX_SEP_RADIUS + 1];
   int32_t rowi[2 * HIPACC_MAX_SEP_RADIUS + 1];
@@ -162,7 +162,7 @@ int launch_random(void* p, int dt, int stride, int ox, int oy, int w, int h, int
 struct BilatArgs {
   Geom g;
   int ksize;
-  int in_vec_ok, out_vec_ok;
+  int out_vec_ok;
   float k2;                 // -c_r * log2(e)
   double scale;             // sqrt(c_r * log2(e)) of the float sigma_r
   float lsp[kMaxTaps];      // log2(spatial)

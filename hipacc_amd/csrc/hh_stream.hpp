@@ -486,7 +486,7 @@ __global__ __launch_bounds__(256) void stream_kernel(const ArgsT a, const Stream
   }
 }
 
-// Alignment the streaming kernels need: V-pixel loads and stores.
+// Whether every row starts on a whole V-pixel vector (at most 16 bytes).
 static inline void stream_align(const Geom& g, int v, int& in_ok, int& out_ok) {
   const int ebi = dtype_bytes(g.in_dtype), ebo = dtype_bytes(g.out_dtype);
   const int ai = v * ebi < 16 ? v * ebi : 16, ao = v * ebo < 16 ? v * ebo : 16;
@@ -536,7 +536,8 @@ static int launch_stream(const ArgsT& a0, int seg_rows, hipStream_t s) {
       (std::is_same<TO, float>::value && a0.g.cvt == HIPACC_CVT_ROUND))
     return HIPACC_ERR_UNSUPPORTED;
   ArgsT a = a0;
-  stream_align(a.g, V, a.in_vec_ok, a.out_vec_ok);
+  int in_ok;   // (rows are loaded at any alignment)
+  stream_align(a.g, V, in_ok, a.out_vec_ok);
   StreamGeom sg = stream_geom(a.g, KX / 2 * CH, V, seg_rows);
   const dim3 grid = stream_grid(sg);
   hipLaunchKernelGGL((stream_kernel<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, ArgsT>), grid,

@@ -18,13 +18,6 @@
 
 namespace hh {
 
-template <int BYTES> struct word_of;
-template <> struct word_of<1> { using type = uint8_t; };
-template <> struct word_of<2> { using type = uint16_t; };
-template <> struct word_of<4> { using type = uint32_t; };
-template <> struct word_of<8> { using type = uint2; };
-template <> struct word_of<16> { using type = uint4; };
-
 // Words of row pixels at any pixel's alignment: global accesses of 4 to 16
 // bytes need none on this device (a wave's row costs at most one more cache
 // line), so rows of odd pitch move as whole vectors too.

@@ -144,7 +144,8 @@ static int launch_ring_sep(const SepArgs& a0, int seg_rows, hipStream_t s) {
     return cus * (per_cu < 3 ? per_cu : 3);
   }();
   SepArgs a = a0;
-  stream_align(a.g, kRingV, a.in_vec_ok, a.out_vec_ok);
+  int in_ok;   // (rows are staged at any alignment)
+  stream_align(a.g, kRingV, in_ok, a.out_vec_ok);
   const long long strips = ceil_div(a.g.is_w, (64 - 2 * HL) * kRingV);
   if (strips * a.g.is_h * a.g.batch > (1ll << 31))
     return set_error(HIPACC_ERR_UNSUPPORTED, "ring_sep kernel: %lld strip rows",
