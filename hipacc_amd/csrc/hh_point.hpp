@@ -31,7 +31,12 @@ template <> __device__ __forceinline__ int32_t point_eval<int32_t>(int op, int32
     case HIPACC_POINT_ADD: return (int32_t)((uint32_t)a + (uint32_t)b);
     case HIPACC_POINT_SUB: return (int32_t)((uint32_t)a - (uint32_t)b);
     case HIPACC_POINT_MUL: return (int32_t)((uint32_t)a * (uint32_t)b);
-    case HIPACC_POINT_ABSDIFF: return a > b ? a - b : b - a;
+    case HIPACC_POINT_ABSDIFF: {
+      // the difference wraps, and the magnitude of INT_MIN is INT_MIN (as
+      // signed expressions the compiler may take either for positive)
+      const uint32_t d = (uint32_t)a - (uint32_t)b;
+      return (int32_t)((int32_t)d < 0 ? 0u - d : d);
+    }
     case HIPACC_POINT_MIN: return a < b ? a : b;
     case HIPACC_POINT_MAX: return a > b ? a : b;
     default: return a;
@@ -54,7 +59,7 @@ __device__ __forceinline__ TO point_pixel(int op, float af, float bf, int32_t ai
       const int32_t nrm = (int32_t)alpha;
       const int32_t q0 = nrm ? ai / nrm : ai;
       const int32_t q1 = nrm ? bi / nrm : bi;
-      float f = sqrtf((float)(q0 * q0 + q1 * q1));
+      float f = sqrtf((float)(int32_t)((uint32_t)q0 * (uint32_t)q0 + (uint32_t)q1 * (uint32_t)q1));
       f = f < 255.0f ? f : 255.0f;
       f = f > 0.0f ? f : 0.0f;
       return convert_f<TO>(f, cvt, 0.0f);

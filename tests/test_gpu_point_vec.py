@@ -53,3 +53,20 @@ def test_magnitude_without_division(gpu, norm):
                          alpha=float(norm), cvt=cvt, src_dtype=code,
                          dst_dtype=ob.CODES[np.dtype(tout)])
                 np.testing.assert_array_equal(to_host(dst, tout), ref)
+
+
+def test_absdiff_of_int32_wraps(gpu):
+    """Differences beyond the int32 range wrap, and the magnitude of INT_MIN is
+    INT_MIN, in point calls and in fused chains, also where the result becomes
+    float."""
+    vals = np.array([-2**31, 2**31 - 1, 0, 1, -1, 5], np.int32)
+    a, b = (np.ascontiguousarray(v) for v in np.meshgrid(np.tile(vals, 11), vals))
+    with np.errstate(over="ignore"):
+        ref = np.abs(a - b).astype(np.float32)
+    A, B = to_gpu(a), to_gpu(b)
+    for run in (lambda o: op.point(capi.POINT_ABSDIFF, A, o, B),
+                lambda o: op.fused(A, o, [dict(kind="point", dtype=capi.F32,
+                                               op=capi.POINT_ABSDIFF, in1=B)])):
+        out = torch.empty(a.shape, dtype=torch.float32, device="cuda")
+        run(out)
+        np.testing.assert_array_equal(to_host(out, np.float32), ref)
