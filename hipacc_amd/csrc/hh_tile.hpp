@@ -33,8 +33,9 @@ typedef unsigned short u16_any __attribute__((aligned(1)));
 template <typename TO, int VEC>
 __device__ __forceinline__ void store_vec(TO* dst, const TO (&v)[VEC], bool aligned = true) {
   constexpr int BYTES = VEC * (int)sizeof(TO);
-  // (a macro: a template parameter would drop the types' alignment; the empty
-  // asm keeps the compiler from joining both stores into a plain one)
+  // (a macro: a template parameter would drop the types' alignment; with an
+  // empty asm on either side of it the plain store can neither be hoisted nor
+  // sunk to join the nontemporal one, which would make both plain)
 #define HH_STORE_WORD(W, p, src)                                    \
   {                                                                 \
     W w;                                                            \
@@ -42,6 +43,7 @@ __device__ __forceinline__ void store_vec(TO* dst, const TO (&v)[VEC], bool alig
     if (aligned) {                                                  \
       __builtin_nontemporal_store(w, (W*)(p));                      \
     } else {                                                        \
+      asm volatile("" ::: "memory");                                \
       *(W*)(p) = w;                                                 \
       asm volatile("" ::: "memory");                                \
     }                                                               \
