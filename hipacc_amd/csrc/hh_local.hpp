@@ -148,6 +148,7 @@ struct HistArgs {
   float scale;
   uint32_t* bins;
   uint32_t* partials;   // [blocks][nbins] per-block histograms (workspace)
+  int vec_rows;         // pitched rows are read as 16-byte vectors (set at the launch)
 };
 // Entries of the histogram's partial-bin workspace: blocks * nbins <= this.
 constexpr int kHistPartialEntries = 1 << 18;

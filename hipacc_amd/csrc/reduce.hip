@@ -10,6 +10,8 @@
 // the result, so the result does not depend on scheduling.  (A last-block
 // ticket would need a device-scope release per block, which writes back
 // the L2 of each XCD and costs more than the second launch.)
+#include <algorithm>
+
 #include "hh_tile.hpp"
 
 namespace hh {
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(kHistThreads) void hist_partial_kernel(const HistAr
   } else {
     for (int y = blockIdx.x; y < a.h; y += gridDim.x) {
       const T* row = static_cast<const T*>(a.in) + (long long)(a.oy + y) * a.stride + a.ox;
-      const int nv = a.w / VEC;
+      const int nv = a.vec_rows ? a.w / VEC : 0;
       for (int i = threadIdx.x; i < nv; i += NT) {
         const red_u4 w = reinterpret_cast<const u32x4_any*>(row)[i];
         count(w);
@@ -324,16 +326,30 @@ static int launch_hist_t(const HistArgs& a, int blocks, hipStream_t s) {
   return hip_status(hipGetLastError(), "hist_partial_kernel launch");
 }
 
-int launch_histogram(const HistArgs& a, int dt, hipStream_t s) {
+int launch_histogram(const HistArgs& a0, int dt, hipStream_t s) {
   const int eb = dt == HIPACC_U8 ? 1 : dt == HIPACC_U16 ? 2 : 4;
-  const long long n = (long long)a.w * a.h;
-  // Contiguous windows: about 64 KiB per block (4096^2 u8: 256 blocks,
-  // 9.9 us for both launches; 16, 32 and 128 KiB: 11.2-11.4 us), at most 512
-  // blocks; other windows: one block per row.  blocks * nbins entries must
-  // fit the partials workspace.
-  const bool flat = a.stride == a.w;
-  const long long chunk = 64 * 1024;
-  const long long want = flat ? (n * eb + chunk - 1) / chunk : a.h;
+  const long long n = (long long)a0.w * a0.h;
+  // Contiguous windows: 64 KiB per block once that makes enough of them (4096^2
+  // u8, 256 bins: 256 blocks, 9.4 us for both launches; 16 KiB: 11.9); smaller
+  // ones 16 and 4 KiB, up to 192 and 64 blocks (us at 64, 16 and 4 KiB, u8:
+  // 333x260, 4096 bins 16.6, 9.5 and 7.3; 1001x751, 1000 bins 11.8, 7.0 and
+  // 7.3; 525x3520, 1000 bins 11.9, 7.4 and 9.0).  Other windows: one block per
+  // row.  At most 512 blocks, and blocks * nbins entries must fit the partials
+  // workspace.
+  const bool flat = a0.stride == a0.w;
+  const long long kib = (n * eb + 1023) / 1024;
+  const long long c64 = (kib + 63) / 64, c16 = (kib + 15) / 16, c4 = (kib + 3) / 4;
+  const long long want =
+      flat ? std::max(c64, std::max(std::min(c16, 192ll), std::min(c4, 64ll))) : a0.h;
+  // Pitched rows as vectors where they are aligned, or so wide that a row keeps
+  // enough of the threads busy (u8 rows, pixels and vectors, 4096 bins:
+  // 256x1868 14.0 and 26.2 us, 1921x1081 18.9 and 20.3, 4031x3023 68.8 and
+  // 57.6; f32 1001x751 12.7 and 13.5, 1500x1500 22.0 and 16.4).
+  HistArgs a = a0;
+  const uintptr_t base =
+      reinterpret_cast<uintptr_t>(a.in) + ((long long)a.oy * a.stride + a.ox) * eb;
+  a.vec_rows = (base % 16 == 0 && (long long)a.stride * eb % 16 == 0) ||
+               a.w >= (eb == 4 ? 1200 : 2048);
   long long blocks = want < 512 ? want : 512;
   const long long cap = kHistPartialEntries / a.nbins;
   if (blocks > cap) blocks = cap;

@@ -124,3 +124,28 @@ def test_global_operators_unaligned(gpu, dtype):
                 np.testing.assert_array_equal(to_host(bins, np.int32),
                                               np.bincount(src.astype(np.int64).ravel(),
                                                           minlength=256))
+
+
+@pytest.mark.parametrize("dt", [np.uint8, np.float32])
+@pytest.mark.parametrize("nbins", [256, 4096])
+def test_histogram_routes(gpu, dt, nbins):
+    """Contiguous windows around the sizes where the share of a block changes,
+    and pitched rows, aligned or not, on either side of the widths that are
+    read as vectors."""
+    eb = np.dtype(dt).itemsize
+    shapes = [(1, n // eb) for n in (4095, 4100, 64 * 4096 + 4, 192 * 16384 - 4, 192 * 65536 + 4)]
+    shapes += [(h, w) for w in (15, 1199, 1200, 2047, 2048, 2049) for h in (3, 700)]
+    for h, w in shapes:
+        a = ob.random_image((h, w), dt, w + nbins)
+        scale = float(nbins) if dt == np.float32 else 1.0
+        ref = ob.histogram(a, nbins, scale)
+        for x0, pad in ((0, 0), (1, 0), (1, 2), (16, 16 + -w % 16)):
+            bins = torch.full((nbins,), -1, dtype=torch.int32, device="cuda")
+            if pad:
+                src = _cut(a, x0, pad)
+            else:   # rows back to back, the first one x0 pixels into the buffer
+                flat = torch.zeros(h * w + x0, dtype=DT[a.dtype], device="cuda")
+                flat[x0:] = to_gpu(a).reshape(-1)
+                src = flat[x0:].view(h, w)
+            op.histogram(src, nbins, bins, scale=scale)
+            np.testing.assert_array_equal(to_host(bins, np.uint32), ref, err_msg=f"{h}x{w} {x0} {pad}")
