@@ -126,6 +126,7 @@ struct PointArgs {
   int op, cvt;
   float alpha, beta;
   int vec_ok;   // output vectors are aligned (set at the launch)
+  int lanes;    // log2 of a block's threads side by side (set at the launch)
 };
 int launch_point(const PointArgs& a, int dt0, int dt1, int dto, hipStream_t s);
 

@@ -12,23 +12,35 @@
 
 namespace hh {
 
-// N pixels at any alignment as one load of up to 16 bytes; only n of them
-// exist when n < N.
-template <typename T, int N> __device__ __forceinline__ void load_n(const T* p, T (&v)[N], int n) {
+template <typename T, int N> __device__ __forceinline__ void load_word(const T* p, T* v) {
   constexpr int B = N * (int)sizeof(T);
-  if (n == N) {
 #define HH_LOAD_WORD(W)                                \
   {                                                    \
     const W w = *reinterpret_cast<const W*>(p);        \
     __builtin_memcpy(v, &w, B);                        \
   }
-    if constexpr (B == 16) HH_LOAD_WORD(u32x4_any)
-    else if constexpr (B == 8) HH_LOAD_WORD(u32x2_any)
-    else HH_LOAD_WORD(u32_any)
+  if constexpr (B == 16) HH_LOAD_WORD(u32x4_any)
+  else if constexpr (B == 8) HH_LOAD_WORD(u32x2_any)
+  else HH_LOAD_WORD(u32_any)
 #undef HH_LOAD_WORD
-  } else {
+}
+
+// N pixels at any alignment as one load of up to 16 bytes; where only n < N of
+// them exist, by fours as far as they go (a wave that holds a row's end waits
+// for these too: u8 magnitude at 712x2050, pitched, 5.4 us pixel by pixel).
+template <typename T, int N> __device__ __forceinline__ void load_n(const T* p, T (&v)[N], int n) {
+  if (n == N) {
+    load_word<T, N>(p, v);
+    return;
+  }
 #pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = k < n ? p[k] : T(0);
+  for (int g = 0; g < N; g += 4) {
+    if (g + 4 <= n) {
+      load_word<T, 4>(p + g, v + g);
+    } else {
+#pragma unroll
+      for (int k = g; k < g + 4; ++k) v[k] = k < n ? p[k] : T(0);
+    }
   }
 }
 
@@ -76,9 +88,10 @@ template <typename T, typename TO>
 __global__ __launch_bounds__(256) void point_kernel(const PointArgs a) {
   constexpr int N = point_pixels<T, TO>();
   constexpr bool FM = std::is_same<T, float>::value;
-  const int x = (blockIdx.x * 256 + threadIdx.x) * N;
-  const int y = blockIdx.y;
-  if (x >= a.w) return;
+  // 2^lanes threads of the block side by side, 256 >> lanes rows
+  const int x = ((int)(blockIdx.x << a.lanes) + (int)(threadIdx.x & ((1 << a.lanes) - 1))) * N;
+  const int y = (int)(blockIdx.y << (8 - a.lanes)) + (int)(threadIdx.x >> a.lanes);
+  if (x >= a.w || y >= a.h) return;
   const int n = a.w - x < N ? a.w - x : N;
   const long long b = blockIdx.z;
   T v0[N], v1[N];
@@ -119,8 +132,16 @@ __global__ __launch_bounds__(256) void point_kernel(const PointArgs a) {
     store_vec<TO, N>(po, r, a.vec_ok);
   } else {
 #pragma unroll
-    for (int k = 0; k < N; ++k)
-      if (k < n) po[k] = r[k];
+    for (int g = 0; g < N; g += 4) {
+      const TO q[4] = {r[g], r[g + 1], r[g + 2], r[g + 3]};
+      if (g + 4 <= n) {
+        store_vec<TO, 4>(po + g, q, false);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (g + k < n) po[g + k] = q[k];
+      }
+    }
   }
 }
 
@@ -141,7 +162,10 @@ static int launch_point_t(const PointArgs& a0, hipStream_t s) {
   const long long align = N * (long long)sizeof(TO);
   a.vec_ok = po % align == 0 && (a.h == 1 || (a.stride_out * (long long)sizeof(TO)) % align == 0) &&
              (a.batch == 1 || (a.plane_out * (long long)sizeof(TO)) % align == 0);
-  dim3 grid(ceil_div(a.w, 256 * N), a.h, a.batch);
+  // blocks of several rows where a row has less than 256 vectors (int8
+  // magnitude, 2 x 128x1840: 7.2 us with 8 of a block's threads in use)
+  while (a.lanes < 8 && (N << a.lanes) < a.w) ++a.lanes;
+  dim3 grid(ceil_div(a.w, N << a.lanes), ceil_div(a.h, 256 >> a.lanes), a.batch);
   hipLaunchKernelGGL((point_kernel<T0, TO>), grid, dim3(256), 0, s, a);
   return hip_status(hipGetLastError(), "point_kernel launch");
 }

@@ -70,3 +70,23 @@ def test_absdiff_of_int32_wraps(gpu):
         out = torch.empty(a.shape, dtype=torch.float32, device="cuda")
         run(out)
         np.testing.assert_array_equal(to_host(out, np.float32), ref)
+
+
+@pytest.mark.parametrize("tin,tout", [(np.uint8, np.uint8), (np.int16, np.float32)])
+def test_point_blocks_of_several_rows(gpu, tin, tout):
+    """Rows of fewer than 256 vectors share a block: widths around 2^k vectors,
+    heights around the block's rows, tails of every kind of length."""
+    kw = dict(src_dtype=ob.CODES[np.dtype(tin)], dst_dtype=ob.CODES[np.dtype(tout)])
+    n = 16 // max(np.dtype(tin).itemsize, np.dtype(tout).itemsize)
+    for vecs in (1, 2, 8, 45, 128, 256):
+        for w in (n * vecs - 1, n * vecs, n * vecs + 1, n * vecs + n // 2):
+            rows = 256 >> min(8, int(np.ceil(np.log2(max(1, -(-w // n))))))
+            for h in (1, rows, 2 * rows + 1):
+                a, b = (ob.random_image((h, w), tin, s + w) for s in (3, 4))
+                ref = np.zeros((h, w), tout)
+                ob.point(capi.POINT_SUB, a, ref, b)
+                buf = empty_gpu((h + 1, w + 3), tout, fill=77)
+                op.point(capi.POINT_SUB, to_gpu(a, w + 1), buf[:h, 1:w + 1], to_gpu(b), **kw)
+                np.testing.assert_array_equal(to_host(buf[:h, 1:w + 1], tout), ref)
+                buf[:h, 1:w + 1] = 77
+                assert bool((buf == 77).all())
