@@ -268,16 +268,20 @@ int dispatch_bilat_pair_grad(const BilatGradArgs& a, int* nblocks, hipStream_t s
   const int r = a.ksize / 2, kk = a.ksize * a.ksize;
   if (!a.gx || !a.sym || r < 2 || r > 4) return HIPACC_ERR_UNSUPPORTED;
   if (!(a.scale > 1e-15 && a.scale < 1e15)) return HIPACC_ERR_UNSUPPORTED;   // as forward
-  // Issue slots of a SIMD, both ways, as in dispatch_bilat_pair (us, tile and
-  // pair): 5x5 at 1024^2 20.1 and 23.4, at 1920x1080 36.0 and 34.0, at 1500^2
-  // 37.4 and 36.3; 7x7 at 1001x751 25.5 and 28.2, at 1920x1080 56.5 and 49.6,
-  // at 2048^2 98 and 82; 9x9 at 1024^2 40.6 and 43.0, at 1500^2 79.5 and 74.4.
-  const double tile = (double)ceil_div(a.ntiles, cus) * (52.0 * kk + 900.0);
-  const double row = 34.0 * kk + 300.0, first = 4000.0;
+  // Issue slots of a SIMD, both ways, as in dispatch_bilat_pair; a single round
+  // of blocks, two waves a SIMD at most, waits for 600 slots a row (us, tile
+  // and pair): 5x5 at 419x2622 22.4 and 23.8, at 2 x 384x3552 39.6 and 44.2, at
+  // 1500^2 37.4 and 36.3; 7x7 at 1001x751 25.5 and 28.2, at 1920x1080 56.5 and
+  // 49.6, at 2048^2 98 and 82; 9x9 at 1024^2 40.6 and 43.0, at 365x3458 48.9
+  // and 49.5, at 1500^2 79.5 and 74.4.
+  const double tile = (double)ceil_div(a.ntiles, cus) * (54.0 * kk + 900.0);
+  const double row = 33.0 * kk + 300.0, first = 1500.0, alone = 600.0;
   if (tile < (kPairRows + 1.0) * row + first) return HIPACC_ERR_UNSUPPORTED;
   const PairGeom pg = pair_geom(a.w, a.h, a.batch, r, cus, kGradBlocks);
   if (pg.blocks == 0) return HIPACC_ERR_UNSUPPORTED;
-  if (tile < ceil_div(pg.blocks, cus) * (pg.n + 1.0) * row + first) return HIPACC_ERR_UNSUPPORTED;
+  const int rounds = ceil_div(pg.blocks, cus);
+  if (tile < rounds * (pg.n + 1.0) * (row + (rounds == 1 ? alone : 0.0)) + first)
+    return HIPACC_ERR_UNSUPPORTED;
   switch (r) {
     case 2: hipLaunchKernelGGL((bilat_pair_grad_kernel<2>), dim3(pg.blocks), dim3(256), 0, s, a, pg); break;
     case 3: hipLaunchKernelGGL((bilat_pair_grad_kernel<3>), dim3(pg.blocks), dim3(256), 0, s, a, pg); break;
