@@ -538,6 +538,13 @@ static int launch_stream(const ArgsT& a0, int seg_rows, hipStream_t s) {
   ArgsT a = a0;
   int in_ok;   // (rows are loaded at any alignment)
   stream_align(a.g, V, in_ok, a.out_vec_ok);
+  // Outputs below 1 MiB take plain stores: the kernel ends with its last store,
+  // which the L2 takes sooner (us, plain and nontemporal: u8 5x5 at 256^2 6.2
+  // and 6.7, at 1024^2 8.4 and 8.6; u8 3x3 MIN at 512^2 5.0 and 5.2, at 4096^2
+  // 16.0 and 14.1; f32 3x3 MIN at 256^2 5.2 and 5.7, at 2880x2160 16.3 and
+  // 14.3; float4 3x3 at 1024^2 10.7 and 9.3).
+  a.out_vec_ok = a.out_vec_ok &&
+                 (long long)a.g.is_w * a.g.is_h * a.g.batch * (long long)sizeof(TO) >= (1 << 20);
   StreamGeom sg = stream_geom(a.g, KX / 2 * CH, V, seg_rows);
   const dim3 grid = stream_grid(sg);
   hipLaunchKernelGGL((stream_kernel<TI, TO, ACC, V, KX, KY, PF, FMA, KIND, WDEV, CH, ArgsT>), grid,

@@ -134,7 +134,8 @@ def test_images_of_a_batch_in_different_units(gpu, train):
 
 @pytest.mark.parametrize("train", [False, True])
 @pytest.mark.parametrize("offset,sigma", [(1000.0, 0.1), (1000.0, 0.01), (0.0, 1e-3),
-                                          (0.0, 1e4), (0.0, 1e12)])
+                                          (0.0, 1e4), (0.0, 1e12), (0.0, 1e-8),
+                                          (0.0, 1e-12)])
 def test_offset_and_sigma(gpu, offset, sigma, train):
     _check(_base(SHAPE, 4) + offset, 7, sigma, capi.REPEAT, 0.0, train)
 
