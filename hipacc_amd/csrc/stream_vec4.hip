@@ -7,7 +7,7 @@
 // float4, and MIN / MAX over whole masks.  The other shapes stay with
 // local_vec4_kernel, which evaluates every tap from an LDS tile of 16-byte
 // pixels with run-time types and mask. 1920x1080 uchar4 5x5: 107 us there,
-// 18.7 us here, where a tap is one FMA per channel (100 FMA per pixel, 5.3 us
+// 18.9 us here, where a tap is one FMA per channel (100 FMA per pixel, 5.3 us
 // of VALU issue, and a third more rows for the segments' halo).
 #include "hh_stream.hpp"
 
